@@ -120,7 +120,6 @@ struct Slot {
     // order (kvals64, kvals32) are copies remade after a write of the slot:
     // they are current when their generation equals gen.
     bool has_plan = false;
-    int32_t sreg = 0;
     DevBuf sched, kperm, kcol, kxrow, kvals64, kvals32;
     uint64_t kvals64_gen = 0, kvals32_gen = 0;
     // blocks in every block row when they are all equal (0: ragged)
@@ -310,7 +309,6 @@ BsrDev dev_view(const Slot &s, bool fp32) {
         d.vals = fp32 ? s.kvals32.p : s.kvals64.p;
         d.xrow = static_cast<const int32_t *>(s.kxrow.p);
         d.sched = static_cast<const int32_t *>(s.sched.p);
-        d.sreg = s.sreg;
         return d;
     }
     d.col_ind = static_cast<const int32_t *>(s.col_ind.p);
@@ -481,8 +479,8 @@ MfmaPlan mfma_plan(int64_t n, const int64_t *rp, const int32_t *ci, int32_t sreg
     return pl;
 }
 
-// Gather table (see BsrDev::xrow) of a real slot with b >= 8, the blocks the
-// MFMA SpMM takes; kXrowSpare trailing entries keep the steps it fetches past
+// Gather table (see BsrDev::xrow) of a slot with b >= 8, the blocks the MFMA
+// SpMM takes, and the plan of a real one; kXrowSpare trailing entries keep the steps it fetches past
 // the last row's K in range.
 int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     s.has_xrow = false;
@@ -493,7 +491,7 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
         while (r < s.nbr && rp[r + 1] - rp[r] == rp[1]) ++r;
         if (r == s.nbr) s.ulen = (int32_t)rp[1];
     }
-    if (s.b < 8 || s.is_complex) return RG_OK;
+    if (s.b < 8) return RG_OK;
     const int64_t n = s.nnzb * s.b;
     if ((int64_t)s.nbr * s.b > INT32_MAX) return RG_OK;
     std::vector<int32_t> t((size_t)n + kXrowSpare, 0);
@@ -502,7 +500,7 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     RG_HIP(ctx, s.xrow.ensure(t.size() * 4), "hipMalloc gather table");
     RG_HIP(ctx, hipMemcpy(s.xrow.p, t.data(), t.size() * 4, hipMemcpyHostToDevice), "upload gather table");
     s.has_xrow = true;
-    if (!ctx->mfma_plan || s.nnzb >= INT32_MAX || s.nbr >= INT32_MAX) return RG_OK;
+    if (!ctx->mfma_plan || s.is_complex || s.nnzb >= INT32_MAX || s.nbr >= INT32_MAX) return RG_OK;
     const int32_t sreg = ctx->mfma_sreg > 0 ? (int32_t)std::min<int64_t>(ctx->mfma_sreg, s.nbr) : plan_region_rows(s.nbr);
     MfmaPlan pl = mfma_plan(s.nbr, rp, ci, sreg);
     std::vector<int32_t> kc((size_t)s.nnzb + 1, 0);
@@ -520,7 +518,6 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
                "upload plan");
     RG_HIP(ctx, hipMemcpy(s.kcol.p, kc.data(), kc.size() * 4, hipMemcpyHostToDevice), "upload plan");
     RG_HIP(ctx, hipMemcpy(s.kxrow.p, t.data(), t.size() * 4, hipMemcpyHostToDevice), "upload plan");
-    s.sreg = pl.sreg;
     s.kvals64_gen = s.kvals32_gen = 0;
     s.has_plan = true;
     return RG_OK;
@@ -1057,7 +1054,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
         for (int sl = 0; sl < (ctx->form == RG_FORM_SANDWICH ? 3 : 1); ++sl) {
             const BsrDev q = dev_view(ctx->slots[sl], vm.fp32);
             for (uint64_t x : {addr(q.row_ptr), addr(q.col_ind), addr(q.vals), addr(q.xrow), addr(q.sched),
-                               (uint64_t)q.sreg, (uint64_t)q.ulen, (uint64_t)q.nbr, (uint64_t)q.b, (uint64_t)q.nnzb,
+                               (uint64_t)q.ulen, (uint64_t)q.nbr, (uint64_t)q.b, (uint64_t)q.nnzb,
                                (uint64_t)q.is_complex})
                 key.push_back(x);
         }
@@ -1238,14 +1235,6 @@ int rg_create(int device_id, rg_context **out) {
     if (const char *v = std::getenv("RG_GRAD_WIDE")) set_grad_wide(std::atoi(v));
     if (const char *v = std::getenv("RG_MFMA_PLAN")) ctx->mfma_plan = std::atoi(v) != 0;
     if (const char *v = std::getenv("RG_MFMA_SREG")) ctx->mfma_sreg = std::max(0, std::atoi(v));
-    if (const char *v = std::getenv("RG_MFMA_PD16")) {
-        // "fp64 plain, fp64 step, fp32 plain, fp32 step"
-        int p[4] = {0, 0, 0, 0};
-        if (std::sscanf(v, "%d,%d,%d,%d", &p[0], &p[1], &p[2], &p[3]) == 4)
-            for (int q = 0; q < 4; ++q) set_mfma_pd16(q / 2, q % 2, p[q]);
-    }
-    if (const char *v = std::getenv("RG_MFMA_PD32")) set_mfma_pd32(std::atoi(v));
-    if (const char *v = std::getenv("RG_MFMA_PD64")) set_mfma_pd64(std::atoi(v));
     if (const char *v = std::getenv("RG_KG_WIDEN_BYTES")) {
         const long long n = std::atoll(v);
         if (n > 0) ctx->kg_widen_bytes = (size_t)n;

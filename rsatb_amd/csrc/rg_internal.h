@@ -8,7 +8,7 @@ namespace rg {
 
 // Spare (zero) entries after the MFMA SpMM's gather table: a wave fetches up
 // to 2 PD - 2 steps of 4 entries past its row, and reads the entries of the
-// step after its last fetch (PD <= 6: at most 8 PD - 2 = 46 entries).
+// step after its last fetch (PD <= 8: at most 8 PD - 2 = 62 entries).
 constexpr int kXrowSpare = 64;
 
 // Device view of one BSR operand. Values are real (vals) or complex
@@ -21,14 +21,12 @@ struct BsrDev {
     const int32_t *col_ind = nullptr;
     const void *vals = nullptr; // double / double2 / float / float2
     bool is_complex = false;
-    // gather table of real b >= 8 matrices, or null: xrow[s * b + kk] =
+    // gather table of b >= 8 matrices, or null: xrow[s * b + kk] =
     // col_ind[s] * b + kk, the X row of column kk of block s (kXrowSpare spare entries)
     const int32_t *xrow = nullptr;
     // processing order of the block rows (MFMA SpMM), or null for stored
-    // order: position p of [0, nbr) computes block row sched[p]. The XCD
-    // ranges of a launch are whole regions of sreg consecutive positions.
+    // order: position p of [0, nbr) computes block row sched[p]
     const int32_t *sched = nullptr;
-    int32_t sreg = 0;
     // > 0 when every block row holds exactly ulen blocks and row_ptr[0] = 0:
     // row br's blocks are then br * ulen .. br * ulen + ulen - 1, and the VALU
     // SpMM computes them instead of loading row_ptr
@@ -91,11 +89,6 @@ void set_b1_slab_min_grid(int g);
 // sample columns a lane (1, 2 or 4; anything else: 2) in the gradient
 // accumulation for 8 < R <= 32
 void set_grad_wide(int cols);
-void set_mfma_pd32(int p);
-void set_mfma_pd64(int p);
-// prefetch depth (2 .. 6) of the sixteen-tile complex MFMA SpMM for one
-// precision and kind (plain product or step)
-void set_mfma_pd16(int fp32, int step, int p);
 
 // Device matrices hold every b x b block column-major; uploads arrive
 // row-major (rsatb's layout) and are transposed on the device.
@@ -109,6 +102,35 @@ int spmm_launch_grid(const BsrDev &A, VecMode vm, int R);
 // Y = epilogue(A X). X, Y: [nbr*b][R] in the storage `vm` describes.
 hipError_t launch_spmm(const BsrDev &A, VecMode vm, const void *X, void *Y, int R,
                        const EpiArgs &e, hipStream_t stream, int *grid_out);
+
+// ---- MFMA SpMM (rg_mfma.h; one translation unit per launch function) ----
+// Shape of one MFMA SpMM launch: W real columns as nchunks chunks of nt tiles,
+// e columns a lane moves per access, mask when 16 nt nchunks > W.
+struct MfmaShape {
+    int nt = 0; // 0: the launch is not one for this kernel
+    int e = 1;
+    int nchunks = 1;
+    bool mask = false;
+};
+
+struct MfmaKnobs {
+    int xcd_map = 1;  // XCD-contiguous row ranges (1) or plain round-robin (0)
+    int ntcap = 16;   // upper bound on the tiles one wave owns
+    int grid_cap = 0; // fixed cap on the grid; 0: what is resident
+};
+extern MfmaKnobs g_mfma;
+
+// Set while spmm_launch_grid asks the MFMA dispatch which grid it would take:
+// the launch then reports the grid without launching.
+extern thread_local bool t_mfma_grid_query;
+
+hipError_t launch_mfma_f64(const MfmaShape &s, const BsrDev &A, bool cv, const void *X, void *Y, int W, int R,
+                           const EpiArgs &e, int grid, hipStream_t st, int *grid_out);
+hipError_t launch_mfma_f32(const MfmaShape &s, const BsrDev &A, bool cv, const void *X, void *Y, int W, int R,
+                           const EpiArgs &e, int grid, hipStream_t st, int *grid_out);
+// complex matrix times complex vectors
+hipError_t launch_mfma_cplx(const MfmaShape &s, const BsrDev &A, bool fp32, const void *X, void *Y, int W, int R,
+                            const EpiArgs &e, int grid, hipStream_t st, int *grid_out);
 
 // out[d*R + u] = sum_g partials[(g*ndot + d)*R + u], fixed order.
 hipError_t launch_reduce(const double2 *partials, int ngroups, int ndot, int R, double2 *out,

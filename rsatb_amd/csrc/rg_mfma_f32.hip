@@ -1,0 +1,12 @@
+// MFMA SpMM instances: real matrices, FP32 with compensated FP64 dots (rg_mfma.h).
+#include "rg_mfma.h"
+
+namespace rg {
+
+hipError_t launch_mfma_f32(const MfmaShape &s, const BsrDev &A, bool cv, const void *X, void *Y, int W, int R,
+                           const EpiArgs &e, int grid, hipStream_t st, int *grid_out) {
+    return cv ? by_shape<float, true, false>(s, A, X, Y, W, R, e, grid, st, grid_out)
+              : by_shape<float, false, false>(s, A, X, Y, W, R, e, grid, st, grid_out);
+}
+
+} // namespace rg
