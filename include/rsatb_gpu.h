@@ -252,6 +252,13 @@ RG_API int rg_compute_dos(rg_context *ctx, double emin, double emax, double de, 
 RG_API int rg_kpm_density(const double *mu, int M, const double *x, int64_t nx, double edge_inset,
                    int kernel, double *rho_out);
 
+/* The same for n_sets moment sets on one grid (the projected density has one
+ * per group): mu [n_sets][M] complex, rho_out [n_sets][nx]. Evaluated on the
+ * context's device when there is enough of it, with the results of
+ * rg_kpm_density bit for bit. */
+RG_API int rg_kpm_density_batch(rg_context *ctx, const double *mu, int64_t n_sets, int M, const double *x,
+                                int64_t nx, double edge_inset, int kernel, double *rho_out);
+
 /* The MFMA SpMM plan the library derives for a square block pattern (real
  * slots with b >= 8 get one at every write): sched_out[nbr] the block rows
  * in processing order (regions of *sreg_out rows, one XCD's rows in flight,

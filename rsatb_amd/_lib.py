@@ -72,6 +72,7 @@ SIGNATURES = {
     "rg_dos_plan": (_i, [_d, _d, _d, C.POINTER(_i), C.POINTER(_i)]),
     "rg_compute_dos": (_i, [_vp, _d, _d, _d, _i, _pd, _pd]),
     "rg_kpm_density": (_i, [_pd, _i, _pd, _i64, _d, _i, _pd]),
+    "rg_kpm_density_batch": (_i, [_vp, _pd, _i64, _i, _pd, _i64, _d, _i, _pd]),
     "rg_mfma_plan": (_i, [_i64, _pi64, _pi32, _pi32, _pi32, C.POINTER(C.c_int32)]),
     "rg_bsr_info": (_i, [_vp, _i, _pi64, C.POINTER(_i), _pi64, C.POINTER(_i)]),
     "rg_download_bsr": (_i, [_vp, _i, _pi64, _pi32, _pd]),
@@ -450,6 +451,17 @@ class Context:
         )
         _check(self._h, rc, "rg_kpm_pdos_moments")
         return total, group
+
+    def kpm_density(self, mu: np.ndarray, x: np.ndarray, edge_inset: float, kernel: int = KERNEL_JACKSON) -> np.ndarray:
+        """evaluate_kpm_density (rsatb/calc/kpm.hpp:206-241) of every row of
+        mu [n_sets, M] on one grid: rho [n_sets, nx]."""
+        mu = np.ascontiguousarray(np.atleast_2d(np.asarray(mu, dtype=np.complex128)))
+        x = np.ascontiguousarray(np.asarray(x, dtype=np.float64))
+        rho = np.zeros((mu.shape[0], x.shape[0]))
+        rc = self._lib.rg_kpm_density_batch(self._h, _dptr(mu.view(np.float64)), int(mu.shape[0]), int(mu.shape[1]),
+                                            _dptr(x), int(x.shape[0]), float(edge_inset), int(kernel), _dptr(rho))
+        _check(self._h, rc, "rg_kpm_density_batch")
+        return rho
 
     def set_checkpointing(self, stride: int) -> None:
         _check(self._h, self._lib.rg_set_checkpointing(self._h, int(stride)), "rg_set_checkpointing")

@@ -170,6 +170,15 @@ hipError_t launch_group_dots(int64_t nchunks, const int64_t *chunk_ptr, const in
 hipError_t launch_group_finish(int64_t G, const int64_t *grp_chunk, int ndot,
                                const double2 *partial, double2 *out, hipStream_t st);
 
+// ---- density reconstruction (rg_density.hip) ----
+// Moment sets one lane evaluates together (1 or 8); the weights of
+// launch_density are packed [ceil(G / batch)][M][batch].
+int density_batch(int64_t G);
+// rho[g * nx + j] = sum_m w_gm T_m(x_j) / (pi sqrt(max(1e-14, 1 - x_j^2))),
+// x_j clamped to 1 - edge_inset; G <= 65535 * batch
+hipError_t launch_density(const double *w, int64_t G, int M, const double *x, int64_t nx, double edge_inset,
+                          double *rho, hipStream_t st);
+
 // ---- graph-local S^{-1/2} patches (rg_isqrt.hip) ----
 hipError_t launch_patch_gather(int64_t first, int64_t count, int b, const int64_t *row_ptr,
                                const int32_t *col_ind, const double *vals, int ld, double *Y,

@@ -283,8 +283,7 @@ class RSATB:
             self._bind_kpoint(k_idx)
             mu_t, mu_g = self._ctx.kpm_pdos_moments(N, groups.group_of_row, groups.n_groups, prec)
             total[k_idx] = 2.0 * _lib.kpm_density(mu_t, x, 0.5 / nt)
-            for g in range(groups.n_groups):
-                pdos[k_idx, g] = 2.0 * _lib.kpm_density(mu_g[g], x, 0.5 / nt)
+            np.multiply(2.0, self._ctx.kpm_density(mu_g, x, 0.5 / nt), out=pdos[k_idx])
         energy = np.concatenate([(np.arange(nt) - nt) * half / nt + shift, np.arange(nt) * half / nt + shift])
         return {
             "energy": energy, "pdos": pdos, "total": total, "n_group": groups.n_groups,
