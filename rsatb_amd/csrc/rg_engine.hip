@@ -635,7 +635,8 @@ struct GroupDots {
     const int64_t *chunk_ptr = nullptr; // [nchunks + 1] into rows
     const int32_t *rows = nullptr;      // rows of group 0, then group 1, ...
     const int64_t *grp_chunk = nullptr; // [G + 1] into chunks
-    double2 *partial = nullptr;         // [nchunks][3]
+    double2 *partial = nullptr;         // [steps][nchunks][3], or [nchunks][3] when not deferred
+    bool defer = false;                 // the chunk sums of all steps are finished in one launch
     double2 *out = nullptr;             // [steps][3][G]
     double bytes = 0.0;                 // algorithmic bytes of one launch pair
 };
@@ -649,11 +650,11 @@ int group_dots(rg_context *ctx, const GroupDots &gd, VecMode vm, int R, int ndot
         if (!a || !b) return fail(ctx, RG_ERR_HIP, "hipEventCreate failed");
         RG_HIP(ctx, hipEventRecord(a, ctx->stream), "hipEventRecord");
     }
-    hipError_t he = launch_group_dots(gd.nchunks, gd.chunk_ptr, gd.rows, R, ndot, vm, v0, v1,
-                                      gd.partial, ctx->stream);
-    if (he != hipSuccess) return hipfail(ctx, he, "group dot launch");
-    he = launch_group_finish(gd.G, gd.grp_chunk, ndot, gd.partial,
-                             gd.out + (size_t)step * 3 * gd.G, ctx->stream);
+    double2 *part = gd.partial + (gd.defer ? (size_t)step * 3 * gd.nchunks : 0);
+    hipError_t he = launch_group_dots(gd.nchunks, gd.chunk_ptr, gd.rows, R, ndot, vm, v0, v1, part, ctx->stream);
+    if (he == hipSuccess && !gd.defer)
+        he = launch_group_finish(gd.G, gd.grp_chunk, ndot, part, 0, gd.out + (size_t)step * 3 * gd.G, 0, 1,
+                                 ctx->stream);
     if (he != hipSuccess) return hipfail(ctx, he, "group dot launch");
     if (ctx->prof) {
         RG_HIP(ctx, hipEventRecord(b, ctx->stream), "hipEventRecord");
@@ -990,7 +991,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     const int chain_slot = ctx->form == RG_FORM_SANDWICH ? RG_SLOT_ZH : RG_SLOT_H;
     const int g_step = spmm_launch_grid(dev_view(ctx->slots[chain_slot], vm.fp32), vm, R);
     const int64_t pstride = (int64_t)g_step * 2 * R; // double2 per step region
-    const bool defer = doubled && !gd && !noalloc && nsteps > 2 &&
+    const bool defer = doubled && !noalloc && nsteps > 2 &&
                        (size_t)nsteps * (size_t)pstride * 16 <= ((size_t)1 << 30);
     double2 *dparts = nullptr;
     if (defer) {
@@ -1136,6 +1137,13 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
             rc = reduce_steps(ctx, g_step, 2, R, raw + (size_t)3 * R, (int64_t)3 * R, dparts + pstride, pstride,
                               nraw - 1);
             if (rc) return rc;
+        }
+        if (gd && gd->defer) { // step 0 left three dots a chunk, the others two
+            hipError_t he = launch_group_finish(gd->G, gd->grp_chunk, 3, gd->partial, 0, gd->out, 0, 1, ctx->stream);
+            if (he == hipSuccess && nraw > 1)
+                he = launch_group_finish(gd->G, gd->grp_chunk, 2, gd->partial + 3 * gd->nchunks, 3 * gd->nchunks,
+                                         gd->out + 3 * gd->G, 3 * gd->G, nraw - 1, ctx->stream);
+            if (he != hipSuccess) return hipfail(ctx, he, "group dot launch");
         }
         rc = rec.end();
         if (rc) return rc;
@@ -1505,8 +1513,11 @@ int rg_kpm_pdos_moments(rg_context *ctx, int M, int precision, int doubling, int
     RG_HIP(ctx, ctx->pd_rows.ensure(rows.size() * 4), "hipMalloc group rows");
     RG_HIP(ctx, ctx->pd_chunk.ensure(chunk_ptr.size() * 8), "hipMalloc group chunks");
     RG_HIP(ctx, ctx->pd_grp.ensure(grp_chunk.size() * 8), "hipMalloc group chunks");
-    RG_HIP(ctx, ctx->pd_partial.ensure((size_t)std::max<int64_t>(nchunks, 1) * 3 * 16),
-           "hipMalloc group partials");
+    // a doubled run keeps every step's chunk dots and finishes them in one
+    // launch (the same sums in the same order) when they fit 1 GiB
+    const size_t part_bytes = (size_t)std::max<int64_t>(nchunks, 1) * 3 * 16;
+    const bool defer = doubled && part_bytes * (size_t)nsteps <= ((size_t)1 << 30);
+    RG_HIP(ctx, ctx->pd_partial.ensure(part_bytes * (defer ? (size_t)nsteps : 1)), "hipMalloc group partials");
     RG_HIP(ctx, ctx->pd_out.ensure((size_t)nsteps * 3 * std::max<int64_t>(G, 1) * 16),
            "hipMalloc group dots");
     RG_HIP(ctx, hipMemcpy(ctx->pd_rows.p, rows.data(), rows.size() * 4, hipMemcpyHostToDevice),
@@ -1525,6 +1536,7 @@ int rg_kpm_pdos_moments(rg_context *ctx, int M, int precision, int doubling, int
     gd.rows = static_cast<const int32_t *>(ctx->pd_rows.p);
     gd.grp_chunk = static_cast<const int64_t *>(ctx->pd_grp.p);
     gd.partial = static_cast<double2 *>(ctx->pd_partial.p);
+    gd.defer = defer;
     gd.out = static_cast<double2 *>(ctx->pd_out.p);
     VecMode vm;
     vm.complex_vec = vec_complex(ctx);

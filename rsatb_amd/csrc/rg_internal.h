@@ -166,9 +166,11 @@ hipError_t launch_group_dots(int64_t nchunks, const int64_t *chunk_ptr, const in
                              int R, int ndot, VecMode vm, const void *v0, const void *v1,
                              double2 *partial, hipStream_t st);
 // out[d * G + g] = sum of group g's chunk partials (chunks grp_chunk[g] ..
-// grp_chunk[g+1]), fixed order.
+// grp_chunk[g+1]), fixed order; nsteps steps in one launch, partial and out
+// advancing by their strides (double2).
 hipError_t launch_group_finish(int64_t G, const int64_t *grp_chunk, int ndot,
-                               const double2 *partial, double2 *out, hipStream_t st);
+                               const double2 *partial, int64_t pstride, double2 *out, int64_t ostride,
+                               int nsteps, hipStream_t st);
 
 // ---- density reconstruction (rg_density.hip) ----
 // Moment sets one lane evaluates together (1 or 8); the weights of

@@ -901,8 +901,10 @@ hipError_t launch_reduce_steps(const double2 *partials, int64_t pstride, int ngr
     // one wave (one dot and column) a workgroup: the strided partial loads
     // spread over as many compute units as there are sums
     const int npairs = ndot * R;
-    hipLaunchKernelGGL(k_reduce, dim3(npairs, (unsigned)nsteps), dim3(64), 0, stream, partials, ngroups, ndot, R,
-                       out, pstride, ostride);
+    for (int s0 = 0; s0 < nsteps; s0 += 65535) // grid.y holds at most 65535
+        hipLaunchKernelGGL(k_reduce, dim3(npairs, (unsigned)std::min(nsteps - s0, 65535)), dim3(64), 0, stream,
+                           partials + (int64_t)s0 * pstride, ngroups, ndot, R, out + (int64_t)s0 * ostride, pstride,
+                           ostride);
     return hipGetLastError();
 }
 
