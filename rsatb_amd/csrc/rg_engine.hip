@@ -124,6 +124,7 @@ struct Slot {
     uint64_t kvals64_gen = 0, kvals32_gen = 0;
     // blocks in every block row when they are all equal (0: ragged)
     int32_t ulen = 0;
+    int32_t maxlen = 0; // most blocks in a block row
     // changes on every write of the slot (context-wide counter), so a pass
     // that keeps state derived from the slot can tell it is stale
     uint64_t gen = 0;
@@ -208,6 +209,10 @@ struct rg_context {
     // replayed moment loops (small operators): the executable graphs of the
     // last captured configuration, one per chunk of steps, and its key
     int graph_mode = 2; // 0 off, 1 always, 2 small operators (RG_GRAPH)
+    // small scalar operators run their moment loop in one launch per column
+    // (the knobs that choose among the launched kernels, RG_GRAPH 0 or 1 and
+    // RG_B1V, ask for those)
+    bool onchip = true;
     // MFMA SpMM plans (row schedule, colour-ordered blocks) for real b >= 8
     // slots written from now on (RG_MFMA_PLAN=0 turns them off)
     bool mfma_plan = true;
@@ -305,6 +310,7 @@ BsrDev dev_view(const Slot &s, bool fp32) {
     d.row_ptr = static_cast<const int64_t *>(s.row_ptr.p);
     d.is_complex = s.is_complex;
     d.ulen = s.ulen;
+    d.maxlen = s.maxlen;
     if (plan_current(s, fp32)) {
         d.col_ind = static_cast<const int32_t *>(s.kcol.p);
         d.vals = fp32 ? s.kvals32.p : s.kvals64.p;
@@ -487,6 +493,9 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     s.has_xrow = false;
     s.has_plan = false;
     s.ulen = 0;
+    int64_t most = 0;
+    for (int64_t r = 0; r < s.nbr; ++r) most = std::max(most, rp[r + 1] - rp[r]);
+    s.maxlen = (int32_t)std::min<int64_t>(most, INT32_MAX);
     if (s.nbr > 0 && rp[0] == 0 && rp[1] > 0 && rp[1] <= 64) {
         int64_t r = 1;
         while (r < s.nbr && rp[r + 1] - rp[r] == rp[1]) ++r;
@@ -888,6 +897,43 @@ struct Recorder {
     }
 };
 
+// Steps one launch of the small-operator loop takes (a few milliseconds).
+constexpr int kOnchipSteps = 8192;
+
+// Downloads the steps' dots and writes the moments (after the loop's launches).
+int finish_moments(rg_context *ctx, int M, int R, int nraw, bool doubled, const double2 *raw, double *mu_out,
+                   double *mu_cols_out, int *nraw_out) {
+    std::vector<double2> host((size_t)nraw * 3 * R);
+    RG_HIP(ctx, hipMemcpyAsync(host.data(), raw, host.size() * sizeof(double2),
+                               hipMemcpyDeviceToHost, ctx->stream),
+           "moment download");
+    RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    if (ctx->prof) drain_events(ctx);
+
+    // per-column moments, then the column mean (dos.hpp:133-138)
+    std::vector<double> mc((size_t)M * R * 2, 0.0);
+    for (int col = 0; col < R; ++col)
+        moments_from_dots(
+            M, nraw, doubled,
+            [&](int step, int d) { return host[((size_t)step * 3 + d) * R + col]; },
+            [&](int m, double2 v) {
+                mc[((size_t)m * R + col) * 2] = v.x;
+                mc[((size_t)m * R + col) * 2 + 1] = v.y;
+            });
+    for (int m = 0; m < M; ++m) {
+        double sr = 0.0, si = 0.0;
+        for (int col = 0; col < R; ++col) {
+            sr += mc[((size_t)m * R + col) * 2];
+            si += mc[((size_t)m * R + col) * 2 + 1];
+        }
+        mu_out[2 * m] = sr / R;
+        mu_out[2 * m + 1] = si / R;
+    }
+    if (mu_cols_out) std::memcpy(mu_cols_out, mc.data(), mc.size() * sizeof(double));
+    if (nraw_out) *nraw_out = nraw;
+    return RG_OK;
+}
+
 // The moment loop of rg_kpm_moments; with gd, the group-resolved dots of
 // every step are written to gd->out as well (steps as moments_from_dots reads
 // them; nraw_out receives the step count).
@@ -991,7 +1037,14 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     const int chain_slot = ctx->form == RG_FORM_SANDWICH ? RG_SLOT_ZH : RG_SLOT_H;
     const int g_step = spmm_launch_grid(dev_view(ctx->slots[chain_slot], vm.fp32), vm, R);
     const int64_t pstride = (int64_t)g_step * 2 * R; // double2 per step region
-    const bool defer = doubled && !noalloc && nsteps > 2 &&
+    const bool keep = doubled && ctx->ckpt_stride > 0 && !vm.fp32 && !noalloc;
+    // Small scalar operators run the whole loop in launches of thousands of
+    // steps. A projected run does so for its all-rows dots (the moments are
+    // those of the plain run bit for bit, for a fraction of a launched step)
+    // and leaves its launched steps unreduced.
+    const bool onchip = ctx->onchip && doubled && !keep && !ctx->prof && ctx->form == RG_FORM_ORTHOGONAL &&
+                        onchip_fits(dev_view(ctx->slots[RG_SLOT_H], vm.fp32), vm);
+    const bool defer = doubled && !onchip && !noalloc && nsteps > 2 &&
                        (size_t)nsteps * (size_t)pstride * 16 <= ((size_t)1 << 30);
     double2 *dparts = nullptr;
     if (defer) {
@@ -1000,7 +1053,6 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     }
 
     // forward states kept for the adjoint: psi_j for j <= 1 and j = 0, K-1 (mod K)
-    const bool keep = doubled && ctx->ckpt_stride > 0 && !vm.fp32 && !noalloc;
     ctx->ckpt_valid = false;
     int Npsi = 1;
     for (int n = 1; 2 * n + 1 < M; ++n) ++Npsi;
@@ -1028,6 +1080,29 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     void *t0 = kept(0) ? kept(0) : wv[0];
     void *t1 = kept(1) ? kept(1) : wv[1];
     void *t2 = wv[2];
+
+    const double a = ctx->half_width, c = ctx->center;
+    if (onchip) { // cancellation is seen between launches
+        rc = stage_samples(ctx, vm, wv[0]);
+        if (rc) return rc;
+        const OnchipWindow win{1.0 / a, -c / a, 2.0 / a, -2.0 * c / a};
+        const int total = std::max(0, (M - 2) / 2); // steps n >= 1 with 2 n + 1 < M
+        int nraw = 0;
+        for (int done = 0; nraw == 0 || done < total;) {
+            const int steps = std::min(total - done, kOnchipSteps);
+            if (ctx->cancel.load()) {
+                (void)hipStreamSynchronize(ctx->stream);
+                return fail(ctx, RG_ERR_CANCELLED, "interrupted");
+            }
+            RG_HIP(ctx, launch_onchip(dev_view(ctx->slots[RG_SLOT_H], vm.fp32), vm, wv[0], wv[1], R, nraw == 0, steps,
+                                      win, raw + (size_t)nraw * 3 * R, ctx->stream),
+                   "moment loop launch");
+            nraw += steps + (nraw == 0 ? 1 : 0);
+            done += steps;
+            if (done < total) RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+        }
+        if (!gd) return finish_moments(ctx, M, R, nraw, true, raw, mu_out, mu_cols_out, nraw_out);
+    }
 
     // graph replay: doubled loops of small operators, outside profiling, the
     // projected moments and the no-allocation entry point (instantiation
@@ -1073,7 +1148,6 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
         RG_HIP(ctx, hipMemcpyAsync(wv[5], t0, nb, hipMemcpyDeviceToDevice, ctx->stream), "psi copy");
     }
 
-    const double a = ctx->half_width, c = ctx->center;
     EpiArgs e;
     e.partials = static_cast<double2 *>(wpart);
 
@@ -1085,7 +1159,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     if (enq) {
         rc = apply_chain(ctx, vm, t0, t1, R, e, &g, -1, zx, hzx);
         if (rc) return rc;
-        rc = reduce(ctx, g, 3, R, raw, parts);
+        if (!onchip) rc = reduce(ctx, g, 3, R, raw, parts);
         if (rc) return rc;
     }
     if (gd) {
@@ -1120,7 +1194,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
                 rc = apply_chain(ctx, vm, t1, t2, R, e, &g, -1, zx, hzx);
                 if (rc) return rc;
                 if (defer && g != g_step) return fail(ctx, RG_ERR_STATE, "step grid differs from its plan");
-                if (!defer) {
+                if (!defer && !onchip) {
                     rc = reduce(ctx, g, 2, R, raw + (size_t)nraw * 3 * R, parts);
                     if (rc) return rc;
                 }
@@ -1183,35 +1257,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
             t2 = sw;
         }
     }
-    std::vector<double2> host((size_t)nraw * 3 * R);
-    RG_HIP(ctx, hipMemcpyAsync(host.data(), raw, host.size() * sizeof(double2),
-                               hipMemcpyDeviceToHost, ctx->stream),
-           "moment download");
-    RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    if (ctx->prof) drain_events(ctx);
-
-    // per-column moments, then the column mean (dos.hpp:133-138)
-    std::vector<double> mc((size_t)M * R * 2, 0.0);
-    for (int col = 0; col < R; ++col)
-        moments_from_dots(
-            M, nraw, doubled,
-            [&](int step, int d) { return host[((size_t)step * 3 + d) * R + col]; },
-            [&](int m, double2 v) {
-                mc[((size_t)m * R + col) * 2] = v.x;
-                mc[((size_t)m * R + col) * 2 + 1] = v.y;
-            });
-    for (int m = 0; m < M; ++m) {
-        double sr = 0.0, si = 0.0;
-        for (int col = 0; col < R; ++col) {
-            sr += mc[((size_t)m * R + col) * 2];
-            si += mc[((size_t)m * R + col) * 2 + 1];
-        }
-        mu_out[2 * m] = sr / R;
-        mu_out[2 * m + 1] = si / R;
-    }
-    if (mu_cols_out) std::memcpy(mu_cols_out, mc.data(), mc.size() * sizeof(double));
-    if (nraw_out) *nraw_out = nraw;
-    return RG_OK;
+    return finish_moments(ctx, M, R, nraw, doubled, raw, mu_out, mu_cols_out, nraw_out);
 }
 
 } // namespace
@@ -1236,7 +1282,9 @@ int rg_create(int device_id, rg_context **out) {
     if (const char *v = std::getenv("RG_GRAPH")) {
         const int m = std::atoi(v);
         ctx->graph_mode = (m == 0 || m == 1) ? m : 2;
+        if (ctx->graph_mode != 2) ctx->onchip = false;
     }
+    if (std::getenv("RG_B1V")) ctx->onchip = false;
     if (const char *v = std::getenv("RG_B1_WIDE")) set_b1_wide(std::atoi(v));
     if (const char *v = std::getenv("RG_ULEN")) set_uniform_rows(std::atoi(v));
     if (const char *v = std::getenv("RG_B1V")) set_b1_slab(std::atoi(v));

@@ -31,6 +31,8 @@ struct BsrDev {
     // row br's blocks are then br * ulen .. br * ulen + ulen - 1, and the VALU
     // SpMM computes them instead of loading row_ptr
     int32_t ulen = 0;
+    // most blocks in a block row
+    int32_t maxlen = 0;
 };
 
 // Epilogue of a SpMM launch. y = sum_blocks A x is finished as
@@ -157,6 +159,20 @@ hipError_t launch_f64_to_f32(const double *in, float *out, int64_t n, hipStream_
 // widening real to complex (zero imaginary part) and/or narrowing to FP32.
 hipError_t launch_stage(const double *in, bool in_complex, void *out, bool out_complex,
                         bool out_fp32, int64_t n, hipStream_t stream);
+
+// ---- moment loop of small scalar operators (rg_onchip.hip) ----
+// Coefficients of t1 = alpha1 A t0 + beta1 t0 and t2 = alpha A t1 + beta t1 - t0.
+struct OnchipWindow {
+    double alpha1, beta1, alpha, beta;
+};
+// b = 1, real matrix, few rows: every column's loop runs in one workgroup
+bool onchip_fits(const BsrDev &A, VecMode vm);
+// `steps` doubled steps in one launch. first: t0 holds the samples, and step 0
+// (t1, <0|0>, <0|1>, <1|1>) comes first; else t0, t1 the state of the launch
+// before. The new state is left in t0, t1 ([rows][R] in the storage of vm);
+// raw: [step][3][R] from the launch's first step on.
+hipError_t launch_onchip(const BsrDev &A, VecMode vm, void *t0, void *t1, int R, bool first, int steps,
+                         const OnchipWindow &w, double2 *raw, hipStream_t st);
 
 // ---- projected moments (rg_pdos.hip) ----
 // partial[c][3] for chunk c = rows[chunk_ptr[c] .. chunk_ptr[c+1]): ndot 1:
