@@ -17,7 +17,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "librsatb_gpu.so"
 
-SOURCES = ["rg_mfma_f64.hip", "rg_mfma_f32.hip", "rg_mfma_cplx.hip", "rg_kernels.hip", "rg_isqrt.hip", "rg_lanczos.hip", "rg_adjoint.hip", "rg_pdos.hip", "rg_density.hip", "rg_onchip.hip",
+SOURCES = ["rg_mfma_f64.hip", "rg_mfma_f32.hip", "rg_mfma_cplx.hip", "rg_kernels.hip", "rg_isqrt.hip", "rg_lanczos.hip", "rg_adjoint.hip", "rg_pdos.hip", "rg_density.hip", "rg_onchip.hip", "rg_kg.hip",
            "rg_sk.hip", "rg_engine.hip"]
 
 # -packed-fp32-ops: hipcc generates no packed (v_pk_*) FP32 arithmetic.

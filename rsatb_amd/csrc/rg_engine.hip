@@ -1950,6 +1950,30 @@ int rg_sk_velocity(rg_context *ctx, const rg_sk_table *t, int64_t n_atoms, const
 
 namespace {
 
+// Whether H and the velocity factors are scalar, real and on one pattern, and
+// the rows whole 16-byte pieces: the sequences then take one launch a moment.
+// With profiling on the products are launched (and timed) one by one.
+int kg_one_pattern(rg_context *ctx, VecMode vm, int R, bool *same) {
+    *same = false;
+    const Slot &H = ctx->slots[RG_SLOT_H];
+    if (H.b != 1 || H.is_complex || ctx->prof || kg_lanes(vm, R) == 0) return RG_OK;
+    for (int a = 0; a < 3; ++a) {
+        const Slot &V = ctx->slots[RG_SLOT_VX + a];
+        if (V.is_complex || V.nnzb != H.nnzb) return RG_OK;
+    }
+    int flag = 0;
+    RG_HIP(ctx, ctx->raw.ensure(16), "hipMalloc flag");
+    RG_HIP(ctx, hipMemcpyAsync(ctx->raw.p, &flag, 4, hipMemcpyHostToDevice, ctx->stream), "clear flag");
+    for (int a = 0; a < 3; ++a)
+        RG_HIP(ctx, launch_same_pattern(dev_view(H, vm.fp32), dev_view(ctx->slots[RG_SLOT_VX + a], vm.fp32),
+                                        static_cast<int *>(ctx->raw.p), ctx->stream),
+               "pattern comparison");
+    RG_HIP(ctx, hipMemcpyAsync(&flag, ctx->raw.p, 4, hipMemcpyDeviceToHost, ctx->stream), "download flag");
+    RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    *same = flag == 0;
+    return RG_OK;
+}
+
 // DC conductivity spectrum (dc_spectrum_fftcheb, rsatb/calc/fftcheb_transport.hpp:
 // 543-653) of the orthogonal form: sigma_out[k * 6 + comp], comp in (xx, xy,
 // xz, yy, yz, zz). Greenwood (formulation 0) fills the diagonal from the
@@ -2035,7 +2059,43 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     // Right: R~_n^a = T_n(A) B_a r; left: L~_n^a = B_a T_n(A) r
     // (fftcheb_transport.hpp:290-430 with V_a = i B_a; the factors -i s of
     // both sides multiply to s^2 in <L|R>)
-    for (int a = 0; a < 3 && !rc; ++a) {
+    bool fused = false;
+    rc = kg_one_pattern(ctx, vm, R, &fused);
+    if (rc) return rc;
+    if (fused) {
+        // scalar operator, one pattern: one launch a moment
+        KgMoment km{};
+        const BsrDev Hd = dev_view(H, fp32);
+        km.h = Hd.vals;
+        for (int a = 0; a < 3; ++a) km.b[a] = dev_view(ctx->slots[RG_SLOT_VX + a], fp32).vals;
+        km.left_stride = km.right_stride = (int64_t)M * nvec;
+        km.alpha1 = first.alpha;
+        km.beta1 = first.beta;
+        km.alpha = step.alpha;
+        km.beta = step.beta;
+        km.cpr = kg_lanes(vm, R);
+        for (int m = 0; m < M; ++m) {
+            km.x = m == 0 ? t0 : t1;
+            km.xp = m == 0 ? nullptr : t0;
+            km.y = m + 1 == M ? nullptr : (m == 0 ? t1 : t2);
+            km.left = Lst(0, m);
+            km.right0 = m == 0 ? Rst(0, 0) : nullptr;
+            km.rx = m >= 1 ? Rst(0, m - 1) : nullptr;
+            km.rxp = m >= 2 ? Rst(0, m - 2) : nullptr;
+            km.ry = m >= 1 ? Rst(0, m) : nullptr;
+            RG_HIP(ctx, launch_kg_moment(Hd, vm, km, m >= 1, ctx->stream), "sequence launch");
+            if (m >= 1 && m + 1 < M) {
+                std::swap(t0, t1); // t0 = T_m r
+                std::swap(t1, t2); // t1 = T_{m+1} r, t2 free
+            }
+            if (ctx->cancel.load()) {
+                (void)hipStreamSynchronize(ctx->stream);
+                drain_events(ctx);
+                return fail(ctx, RG_ERR_CANCELLED, "interrupted");
+            }
+        }
+    }
+    for (int a = 0; a < 3 && !rc && !fused; ++a) {
         rc = spmm(ctx, RG_SLOT_VX + a, vm, t0, Rst(a, 0), R, plain, nullptr);
         if (!rc && M > 1) rc = apply_chain(ctx, vm, Rst(a, 0), Rst(a, 1), R, first, &g);
         for (int n = 2; n < M && !rc; ++n) {
@@ -2049,7 +2109,7 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
         }
     }
     if (rc) return rc;
-    for (int m = 0; m < M && !rc; ++m) {
+    for (int m = 0; m < M && !rc && !fused; ++m) {
         void *bm = t0;
         if (m == 1) {
             rc = apply_chain(ctx, vm, t0, t1, R, first, &g);
@@ -2266,36 +2326,21 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     // node weights (complex, column-major [n + k M]), theta_k = pi (k + 1/2) / M:
     //   GC[n,k] = g_n cos(n theta_k), GE[n,k] = g_n e^{i n theta_k}, GNE = n GE,
     //   g_n = 2 j_n / (pi (1 + delta_n0))    (fftcheb_transport.hpp:259-273)
-    std::vector<double> gw((size_t)M), Wh(3 * zmat, 0.0);
+    std::vector<double> gw((size_t)M);
     for (int n = 0; n < M; ++n) gw[n] = 2.0 * gk[n] / (M_PI * (n == 0 ? 2.0 : 1.0));
-    for (int k = 0; k < M; ++k) {
-        const double th = M_PI * (k + 0.5) / M;
-        for (int n = 0; n < M; ++n) {
-            const size_t o = 2 * ((size_t)k * M + n);
-            Wh[o] = gw[n] * std::cos(n * th);
-            Wh[zmat + o] = gw[n] * std::cos(n * th);
-            Wh[zmat + o + 1] = gw[n] * std::sin(n * th);
-            Wh[2 * zmat + o] = n * gw[n] * std::cos(n * th);
-            Wh[2 * zmat + o + 1] = n * gw[n] * std::sin(n * th);
-        }
-    }
-    RG_HIP(ctx, hipMemcpyAsync(Wz, Wh.data(), Wh.size() * 8, hipMemcpyHostToDevice, ctx->stream),
+    RG_HIP(ctx, ctx->den_in.ensure((size_t)M * 8), "hipMalloc node weights");
+    RG_HIP(ctx, ctx->den_out.ensure((size_t)np * 4 * M * 16), "hipMalloc node sums");
+    RG_HIP(ctx, hipMemcpyAsync(ctx->den_in.p, gw.data(), (size_t)M * 8, hipMemcpyHostToDevice, ctx->stream),
            "upload node weights");
+    RG_HIP(ctx, launch_kg_weights(M, static_cast<const double *>(ctx->den_in.p), reinterpret_cast<double2 *>(Wz),
+                                  ctx->stream),
+           "node weights");
     // sigma from one set of moments (linear in them: the tangent moments give
     // the tangent spectrum)
     auto finish = [&](const double *mu_dev, double *sig_out, double *muh_out) -> int {
-    // complex copies of mu (a real mu widened on the host)
-    std::vector<double> mu_h(mu_real);
-    RG_HIP(ctx, hipMemcpyAsync(mu_h.data(), mu_dev, mu_real * 8, hipMemcpyDeviceToHost, ctx->stream),
-           "download moments");
-    RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    std::vector<double> muz_h((size_t)np * zmat);
-    for (size_t q = 0; q < (size_t)np * mm; ++q) {
-        muz_h[2 * q] = vm.complex_vec ? mu_h[2 * q] : mu_h[q];
-        muz_h[2 * q + 1] = vm.complex_vec ? mu_h[2 * q + 1] : 0.0;
-    }
-    RG_HIP(ctx, hipMemcpyAsync(muz, muz_h.data(), muz_h.size() * 8, hipMemcpyHostToDevice, ctx->stream),
-           "upload moments");
+    // complex copies of mu
+    RG_HIP(ctx, launch_kg_widen(mu_dev, vm.complex_vec, reinterpret_cast<double2 *>(muz), (int64_t)np * mm, ctx->stream),
+           "widen moments");
     // Q_t = mu W_t (Greenwood: t = GC only; Bastin: GE, GC, GNE)
     const int nq = formulation == 1 ? 3 : 1;
     for (int pi = 0; pi < np; ++pi)
@@ -2309,8 +2354,16 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
                 reinterpret_cast<rocblas_double_complex *>(Qz + ((size_t)pi * 3 + t) * zmat), M);
             if (st != rocblas_status_success) return fail(ctx, RG_ERR_HIP, "node GEMM failed");
         }
-    std::vector<double> Qh((size_t)np * 3 * zmat);
-    RG_HIP(ctx, hipMemcpyAsync(Qh.data(), Qz, Qh.size() * 8, hipMemcpyDeviceToHost, ctx->stream), "download");
+    RG_HIP(ctx, launch_kg_nodes(M, formulation == 1, np, reinterpret_cast<const double2 *>(Wz),
+                                reinterpret_cast<const double2 *>(Qz), static_cast<double2 *>(ctx->den_out.p),
+                                ctx->stream),
+           "node sums");
+    std::vector<double> sums((size_t)np * 4 * M * 2), muz_h(muh_out ? (size_t)np * zmat : 0);
+    RG_HIP(ctx, hipMemcpyAsync(sums.data(), ctx->den_out.p, sums.size() * 8, hipMemcpyDeviceToHost, ctx->stream),
+           "download node sums");
+    if (muh_out)
+        RG_HIP(ctx, hipMemcpyAsync(muz_h.data(), muz, muz_h.size() * 8, hipMemcpyDeviceToHost, ctx->stream),
+               "download moments");
     RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     if (ctx->prof) drain_events(ctx);
     if (muh_out) // [pair][m][n] complex, m the left index
@@ -2325,29 +2378,17 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     // kernel_native[k][pair] (divided by the sample count, fftcheb_transport.hpp:595-597)
     std::vector<std::complex<double>> kern((size_t)M * np);
     for (int pi = 0; pi < np; ++pi) {
-        auto Q = [&](int t, int m, int k) {
-            const size_t o = 2 * (((size_t)pi * 3 + t) * mm + (size_t)k * M + m);
-            return std::complex<double>(Qh[o], Qh[o + 1]);
+        auto S = [&](int j, int k) {
+            const size_t o = 2 * (((size_t)pi * 4 + j) * M + k);
+            return std::complex<double>(sums[o], sums[o + 1]);
         };
         for (int k = 0; k < M; ++k) {
             const double th = M_PI * (k + 0.5) / M, eps = std::cos(th);
-            std::complex<double> v(0.0, 0.0);
-            if (formulation == 0) {
-                for (int m = 0; m < M; ++m) v += gw[m] * std::cos(m * th) * Q(0, m, k);
+            std::complex<double> v = S(0, k);
+            if (formulation == 0)
                 v /= std::max(1e-14, 1.0 - eps * eps);
-            } else {
-                // eps (conj(L3) R1 + conj(L1) R3) + i sin (conj(L2) R3 - conj(L3) R2)
-                std::complex<double> l3r1(0.0, 0.0), l1r3(0.0, 0.0), l2r3(0.0, 0.0), l3r2(0.0, 0.0);
-                for (int m = 0; m < M; ++m) {
-                    const double cm = gw[m] * std::cos(m * th);
-                    const std::complex<double> em = gw[m] * std::polar(1.0, -m * th);
-                    l3r1 += cm * Q(0, m, k);
-                    l1r3 += em * Q(1, m, k);
-                    l2r3 += (double)m * em * Q(1, m, k);
-                    l3r2 += cm * Q(2, m, k);
-                }
-                v = eps * (l3r1 + l1r3) + std::complex<double>(0.0, std::sin(th)) * (l2r3 - l3r2);
-            }
+            else // eps (conj(L3) R1 + conj(L1) R3) + i sin (conj(L2) R3 - conj(L3) R2)
+                v = eps * (S(0, k) + S(1, k)) + std::complex<double>(0.0, std::sin(th)) * (S(2, k) - S(3, k));
             kern[(size_t)k * np + pi] = v / (double)R;
         }
     }

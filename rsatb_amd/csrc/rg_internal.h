@@ -278,6 +278,34 @@ hipError_t launch_widen_cols(const float *in, int64_t ld_in, double *out, int64_
 // y = alpha x + beta y over n doubles
 hipError_t launch_axpby(double *y, const double *x, double alpha, double beta, int64_t n, hipStream_t st);
 
+// ---- Kubo-Greenwood sequences of scalar operators (rg_kg.hip) ----
+// One moment m: x = T_m r, xp = T_{m-1} r (null at m = 0); left[d] = B_d x; y =
+// T_{m+1} r unless null; right0[d] = B_d x as well unless null; and, with
+// `right`, ry = R_m from rx = R_{m-1}, rxp = R_{m-2} (null at m = 1) for three
+// axes right_stride apart. Strides in scalars; cpr = kg_lanes().
+struct KgMoment {
+    const void *h, *b[3]; // values on H's pattern
+    const void *x, *xp;
+    void *y, *left, *right0;
+    int64_t left_stride;
+    const void *rx, *rxp;
+    void *ry;
+    int64_t right_stride;
+    double alpha1, beta1, alpha, beta;
+    int cpr;
+};
+// lanes a row takes (whole 16-byte pieces, at most 256), or 0
+int kg_lanes(VecMode vm, int R);
+hipError_t launch_kg_moment(const BsrDev &H, VecMode vm, const KgMoment &a, int right, hipStream_t st);
+// *flag = 1 unless A and B (same rows and entry count) have the same pattern
+hipError_t launch_same_pattern(const BsrDev &A, const BsrDev &B, int *flag, hipStream_t st);
+// node weights GC, GE, GNE ([m + k M] complex each) from the damping g[m]
+hipError_t launch_kg_weights(int M, const double *g, double2 *W, hipStream_t st);
+hipError_t launch_kg_widen(const double *in, bool cplx, double2 *out, int64_t n, hipStream_t st);
+// node sums (see k_kg_nodes): out [npairs][4][M]
+hipError_t launch_kg_nodes(int M, bool bastin, int npairs, const double2 *W, const double2 *Q, double2 *out,
+                           hipStream_t st);
+
 // ---- Slater-Koster assembly (rg_sk.hip) ----
 // Device copy of one matrix's SK table; channels grouped by (row type, col
 // type), pair_ch[2 (rt T + ct)] .. [+1] the range of a pair's channels.

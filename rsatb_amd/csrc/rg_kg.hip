@@ -1,0 +1,243 @@
+// Kubo-Greenwood sequences of a scalar (b = 1, real) operator, and the node
+// sums of the spectrum.
+//
+// One launch a moment in place of seven. The base vector x = T_m r is gathered
+// once for four products, H x (the recurrence) and B_a x (the left vectors),
+// whose matrices share H's pattern, and blockIdx.y adds the three right
+// recurrences, which never meet the base. No dots are formed. A lane owns 16
+// contiguous bytes of a row and a workgroup holds as many whole rows
+// as fit 256 lanes, so any width of whole 16-byte pieces is taken. Every
+// product and recurrence is the launched kernels' operations in their order.
+// Bound: the six vectors a moment that are stored (HBM), and the gather.
+// Measured at graphene 128 x 128 (65,536 rows of four, R = 16, FP64): seven
+// launches 7.5 us each, 52 us a moment; 23 us a moment here (126 MB, 5.5 TB/s).
+#include "rg_internal.h"
+
+#include <type_traits>
+
+namespace rg {
+namespace {
+
+template <typename S> __device__ __forceinline__ S fmas(S a, S b, S c);
+template <> __device__ __forceinline__ double fmas(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <> __device__ __forceinline__ float fmas(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double affine(double v, double alpha, double beta, double s) {
+    return __builtin_fma(alpha, v, beta * s);
+}
+__device__ __forceinline__ float affine(float v, double alpha, double beta, float s) {
+    return (float)__builtin_fma(alpha, (double)v, beta * (double)s);
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void k_kg_moment(int64_t n, int ulen, const int64_t *__restrict__ row_ptr,
+                                                   const int32_t *__restrict__ col_ind, KgMoment a) {
+    constexpr int E = 16 / (int)sizeof(S); // scalars a lane owns
+    typedef S C16 __attribute__((ext_vector_type(E)));
+    const int cpr = a.cpr, rpb = 256 / cpr;
+    const int lr = (int)threadIdx.x / cpr, q = (int)threadIdx.x - lr * cpr;
+    const int64_t br = (int64_t)blockIdx.x * rpb + lr;
+    if (lr >= rpb || br >= n) return;
+    const int64_t W = (int64_t)cpr * E, idx = br * W + (int64_t)q * E;
+    const int64_t s0 = ulen > 0 ? br * ulen : row_ptr[br], s1 = ulen > 0 ? s0 + ulen : row_ptr[br + 1];
+    const S *__restrict__ h = static_cast<const S *>(a.h);
+    auto at = [&](const void *p, int64_t off) -> C16 { return *reinterpret_cast<const C16 *>(static_cast<const S *>(p) + off); };
+    auto put = [&](void *p, C16 v) { *reinterpret_cast<C16 *>(static_cast<S *>(p) + idx) = v; };
+    auto recur = [&](C16 y, const void *x, const void *xp) -> C16 {
+        const C16 xs = at(x, idx);
+        const bool first = xp == nullptr;
+        C16 o;
+#pragma unroll
+        for (int i = 0; i < E; ++i) o[i] = affine(y[i], first ? a.alpha1 : a.alpha, first ? a.beta1 : a.beta, xs[i]);
+        if (!first) {
+            const C16 p = at(xp, idx);
+#pragma unroll
+            for (int i = 0; i < E; ++i) o[i] = o[i] - p[i];
+        }
+        return o;
+    };
+    constexpr int U = 4; // entries whose indices and gathers are in flight together
+    if (blockIdx.y > 0) {
+        // R_m = 2 A~ R_{m-1} - R_{m-2} of one axis
+        const int64_t off = (int64_t)(blockIdx.y - 1) * a.right_stride;
+        const S *x = static_cast<const S *>(a.rx) + off;
+        const S *xp = a.rxp ? static_cast<const S *>(a.rxp) + off : nullptr;
+        C16 y = C16(S(0));
+        int64_t s = s0;
+        for (; s + U <= s1; s += U) {
+            int64_t c[U];
+            S v[U];
+            C16 g[U];
+#pragma unroll
+            for (int t = 0; t < U; ++t) {
+                c[t] = col_ind[s + t];
+                v[t] = h[s + t];
+            }
+#pragma unroll
+            for (int t = 0; t < U; ++t) g[t] = at(x, c[t] * W + (int64_t)q * E);
+#pragma unroll
+            for (int t = 0; t < U; ++t)
+#pragma unroll
+                for (int i = 0; i < E; ++i) y[i] = fmas<S>(v[t], g[t][i], y[i]);
+        }
+        for (; s < s1; ++s) {
+            const C16 g = at(x, (int64_t)col_ind[s] * W + (int64_t)q * E);
+#pragma unroll
+            for (int i = 0; i < E; ++i) y[i] = fmas<S>(h[s], g[i], y[i]);
+        }
+        put(static_cast<S *>(a.ry) + off, recur(y, x, xp));
+        return;
+    }
+    const S *__restrict__ b0 = static_cast<const S *>(a.b[0]), *__restrict__ b1 = static_cast<const S *>(a.b[1]),
+                         *__restrict__ b2 = static_cast<const S *>(a.b[2]);
+    C16 y = C16(S(0)), l0 = y, l1 = y, l2 = y;
+    auto add = [&](C16 g, S vh, S v0, S v1, S v2) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            y[i] = fmas<S>(vh, g[i], y[i]);
+            l0[i] = fmas<S>(v0, g[i], l0[i]);
+            l1[i] = fmas<S>(v1, g[i], l1[i]);
+            l2[i] = fmas<S>(v2, g[i], l2[i]);
+        }
+    };
+    int64_t s = s0;
+    for (; s + U <= s1; s += U) {
+        int64_t c[U];
+        S v[U][4];
+        C16 g[U];
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+            c[t] = col_ind[s + t];
+            v[t][0] = h[s + t];
+            v[t][1] = b0[s + t];
+            v[t][2] = b1[s + t];
+            v[t][3] = b2[s + t];
+        }
+#pragma unroll
+        for (int t = 0; t < U; ++t) g[t] = at(a.x, c[t] * W + (int64_t)q * E);
+#pragma unroll
+        for (int t = 0; t < U; ++t) add(g[t], v[t][0], v[t][1], v[t][2], v[t][3]);
+    }
+    for (; s < s1; ++s) add(at(a.x, (int64_t)col_ind[s] * W + (int64_t)q * E), h[s], b0[s], b1[s], b2[s]);
+    const C16 l[3] = {l0, l1, l2};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        put(static_cast<S *>(a.left) + d * a.left_stride, l[d]);
+        if (a.right0) put(static_cast<S *>(a.right0) + d * a.left_stride, l[d]);
+    }
+    if (a.y) put(a.y, recur(y, a.x, a.xp));
+}
+
+// *flag = 1 unless the two patterns are the same (their row counts are)
+__global__ __launch_bounds__(256) void k_same_pattern(int64_t n, int64_t nnz, const int64_t *__restrict__ rp,
+                                                      const int64_t *__restrict__ rq, const int32_t *__restrict__ cp,
+                                                      const int32_t *__restrict__ cq, int *__restrict__ flag) {
+    bool same = true;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < nnz + n + 1; t += (int64_t)gridDim.x * 256)
+        same = same && (t < nnz ? cp[t] == cq[t] : rp[t - nnz] == rq[t - nnz]);
+    if (!same) *flag = 1;
+}
+
+// Node weights, complex column-major [m + k M], theta_k = pi (k + 1/2) / M:
+// GC = g cos(m theta), GE = g e^{i m theta}, GNE = m GE
+__global__ __launch_bounds__(256) void k_kg_weights(int M, const double *__restrict__ g, double2 *__restrict__ W) {
+    const int64_t mm = (int64_t)M * M;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < mm; t += (int64_t)gridDim.x * 256) {
+        const int m = (int)(t % M), k = (int)(t / M);
+        const double th = 3.14159265358979323846 * (k + 0.5) / M;
+        double sn, cs;
+        sincos(m * th, &sn, &cs);
+        W[t] = double2{g[m] * cs, 0.0};
+        W[mm + t] = double2{g[m] * cs, g[m] * sn};
+        W[2 * mm + t] = double2{m * g[m] * cs, m * g[m] * sn};
+    }
+}
+
+__global__ __launch_bounds__(256) void k_kg_widen(const double *__restrict__ in, int cplx, double2 *__restrict__ out,
+                                                  int64_t n) {
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256)
+        out[t] = cplx ? double2{in[2 * t], in[2 * t + 1]} : double2{in[t], 0.0};
+}
+
+// One wave a node k and pair: the sums over m of (weight column k) x (column k
+// of Q_t). out[(pair * 4 + j) * M + k]: Greenwood j = 0: GC Q_0; Bastin
+// GC Q_0, conj(GE) Q_1, conj(GNE) Q_1, GC Q_2.
+__global__ __launch_bounds__(256) void k_kg_nodes(int M, int bastin, const double2 *__restrict__ W,
+                                                  const double2 *__restrict__ Q, double2 *__restrict__ out) {
+    const int k = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (k >= M) return;
+    const int64_t mm = (int64_t)M * M;
+    const double2 *w = W + (int64_t)k * M, *q = Q + (int64_t)blockIdx.y * 3 * mm + (int64_t)k * M;
+    double2 *o = out + (int64_t)blockIdx.y * 4 * M + k;
+    auto sum = [&](int wsel, bool conj, int t) -> double2 {
+        double2 s{0.0, 0.0};
+        for (int m = lane; m < M; m += 64) {
+            const double2 a = w[wsel * mm + m], b = q[t * mm + m];
+            const double ai = conj ? -a.y : a.y;
+            s.x += a.x * b.x - ai * b.y;
+            s.y += a.x * b.y + ai * b.x;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            s.x += __shfl_xor(s.x, off);
+            s.y += __shfl_xor(s.y, off);
+        }
+        return s;
+    };
+    const double2 a = sum(0, false, 0);
+    if (lane == 0) o[0] = a;
+    if (!bastin) return;
+    const double2 b = sum(1, true, 1), c = sum(2, true, 1), d = sum(0, false, 2);
+    if (lane == 0) {
+        o[M] = b;
+        o[2 * M] = c;
+        o[3 * M] = d;
+    }
+}
+
+unsigned grid_for(int64_t n) {
+    const int64_t g = (n + 255) / 256;
+    return (unsigned)(g < 1 ? 1 : g > 8192 ? 8192 : g);
+}
+
+} // namespace
+
+int kg_lanes(VecMode vm, int R) {
+    const int64_t bytes = (int64_t)R * (vm.complex_vec ? 2 : 1) * (vm.fp32 ? 4 : 8);
+    return bytes % 16 == 0 && bytes <= 16 * 256 ? (int)(bytes / 16) : 0;
+}
+
+hipError_t launch_kg_moment(const BsrDev &H, VecMode vm, const KgMoment &a, int right, hipStream_t st) {
+    if (H.b != 1 || H.is_complex || a.cpr < 1 || a.cpr > 256) return hipErrorInvalidValue;
+    const int rpb = 256 / a.cpr;
+    const dim3 grid((unsigned)((H.nbr + rpb - 1) / rpb), right ? 4 : 1);
+    if (vm.fp32)
+        hipLaunchKernelGGL((k_kg_moment<float>), grid, dim3(256), 0, st, H.nbr, H.ulen, H.row_ptr, H.col_ind, a);
+    else
+        hipLaunchKernelGGL((k_kg_moment<double>), grid, dim3(256), 0, st, H.nbr, H.ulen, H.row_ptr, H.col_ind, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_same_pattern(const BsrDev &A, const BsrDev &B, int *flag, hipStream_t st) {
+    hipLaunchKernelGGL(k_same_pattern, dim3(grid_for(A.nnzb + A.nbr + 1)), dim3(256), 0, st, A.nbr, A.nnzb, A.row_ptr,
+                       B.row_ptr, A.col_ind, B.col_ind, flag);
+    return hipGetLastError();
+}
+
+hipError_t launch_kg_weights(int M, const double *g, double2 *W, hipStream_t st) {
+    hipLaunchKernelGGL(k_kg_weights, dim3(grid_for((int64_t)M * M)), dim3(256), 0, st, M, g, W);
+    return hipGetLastError();
+}
+
+hipError_t launch_kg_widen(const double *in, bool cplx, double2 *out, int64_t n, hipStream_t st) {
+    hipLaunchKernelGGL(k_kg_widen, dim3(grid_for(n)), dim3(256), 0, st, in, cplx ? 1 : 0, out, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_kg_nodes(int M, bool bastin, int npairs, const double2 *W, const double2 *Q, double2 *out,
+                           hipStream_t st) {
+    hipLaunchKernelGGL(k_kg_nodes, dim3((unsigned)((M + 3) / 4), (unsigned)npairs), dim3(256), 0, st, M, bastin ? 1 : 0,
+                       W, Q, out);
+    return hipGetLastError();
+}
+
+} // namespace rg
