@@ -64,6 +64,19 @@ int g_uniform_rows = 1;
 // 25.1 -> 23.7 ms and backward 70.4 -> 69.5 ms against 16 bytes).
 int g_b1v_bytes = -1;
 int g_b1v_min_grid = 512;
+// The same for the slab layout of other widths; long rows (eight entries on
+// average) gain from it down to 256 workgroups. Measured, FP64, column-per-lane
+// against slabs: 16,384 rows of four, R = 10 complex (655 workgroups) 7.1 / 7.7
+// us, R = 24 real (780) 7.4 / 8.0; 65,536 rows, R = 24 15.4 / 11.5; 9,000 rows
+// of thirteen, R = 10 complex (360) 10.0 / 8.0, R = 24 (428) 9.3 / 8.2.
+int g_b1g_min_grid = 1024;
+constexpr int kLongRow = 8, kLongRowMinGrid = 256;
+// Vector bytes up to which the slab SpMMs walk XCD-contiguous row ranges.
+// Measured (round robin / contiguous): 479,596 rows of thirteen, FP32 R = 32
+// (61 MB) 71.9 / 69.0 us, FP64 R = 4 46.2 / 34.3, R = 10 56.7 / 49.2, R = 32
+// complex (245 MB) 302 / 318; 59,212 rows, R = 32 complex (30 MB) 33.7 / 30.8;
+// 1,048,576 rows of four, R = 16 (134 MB) 93.1 / 99.0.
+constexpr int64_t kXcdVectorBytes = (int64_t)64 << 20;
 template <typename S> struct V2;
 template <> struct V2<double> { using T = double2; };
 template <> struct V2<float> { using T = float2; };
@@ -364,6 +377,27 @@ hipError_t by_block(const BsrDev &A, const void *X, void *Y, int R, const EpiArg
     return by_layout<S, CM, CV, 0>(A, X, Y, R, e, grid, st);
 }
 
+// The rows of a workgroup of a grid-stride launch, `per` rows a stride. With
+// xcd (the grid a multiple of 8) every XCD walks its own contiguous eighth:
+// workgroups go to the XCDs in turn, and neighbouring rows gather the same
+// rows of X through one L2.
+struct RowWalk {
+    int64_t lo, hi, step;
+    __device__ __forceinline__ RowWalk(int64_t n, int per, int xcd) {
+        if (xcd) {
+            const int64_t eighth = ((n + per - 1) / per + 7) / 8 * per;
+            const int64_t x0 = (int64_t)(blockIdx.x & 7) * eighth;
+            lo = x0 + (int64_t)(blockIdx.x >> 3) * per;
+            hi = min(n, x0 + eighth);
+            step = (int64_t)(gridDim.x >> 3) * per;
+        } else {
+            lo = (int64_t)blockIdx.x * per;
+            hi = n;
+            step = (int64_t)gridDim.x * per;
+        }
+    }
+};
+
 // ------------------------------------------------------- b = 1 slab SpMM
 // Scalar entries, real matrix, R = LPR * CPL exactly: lane q of a row's LPR
 // lanes owns the contiguous slab of columns q * CPL .. q * CPL + CPL - 1 and
@@ -374,7 +408,7 @@ hipError_t by_block(const BsrDev &A, const void *X, void *Y, int R, const EpiArg
 // in the same order as there (the dots differ only in their summation
 // order). Vector operands must be 16-byte aligned.
 template <typename S, bool CV, int LPR, int CPL>
-__global__ __launch_bounds__(256) void k_spmm_b1v(int64_t nbr, int ulen, const int64_t *__restrict__ row_ptr,
+__global__ __launch_bounds__(256) void k_spmm_b1v(int64_t nbr, int ulen, int xcd, const int64_t *__restrict__ row_ptr,
                                                   const int32_t *__restrict__ col_ind,
                                                   const S *__restrict__ vals, const S *__restrict__ X,
                                                   S *__restrict__ Y, EpiArgs e) {
@@ -417,10 +451,10 @@ __global__ __launch_bounds__(256) void k_spmm_b1v(int64_t nbr, int ulen, const i
 #pragma unroll
         for (int j = 0; j < CPL; ++j) dacc[d][j] = double2{0.0, 0.0};
 
-    const int64_t rows_per_wg = (int64_t)kWaves * G;
-    for (int64_t base = (int64_t)blockIdx.x * rows_per_wg; base < nbr; base += (int64_t)gridDim.x * rows_per_wg) {
+    const RowWalk walk(nbr, kWaves * G, xcd);
+    for (int64_t base = walk.lo; base < walk.hi; base += walk.step) {
         const int64_t br = base + (int64_t)wave * G + g;
-        if (br >= nbr) continue;
+        if (br >= walk.hi) continue;
         S acc[NS];
 #pragma unroll
         for (int i = 0; i < NS; ++i) acc[i] = S(0);
@@ -430,7 +464,7 @@ __global__ __launch_bounds__(256) void k_spmm_b1v(int64_t nbr, int ulen, const i
         int64_t s = s0;
         constexpr int U = 4;
         for (; s + U <= s1; s += U) {
-            int64_t bc[U];
+            int32_t bc[U];
             S a[U];
 #pragma unroll
             for (int t = 0; t < U; ++t) {
@@ -550,6 +584,178 @@ __global__ __launch_bounds__(256) void k_spmm_b1v(int64_t nbr, int ulen, const i
     }
 }
 
+// The slab layout for any row of whole 16-byte pieces: cpr lanes a row (a
+// piece each), as many whole rows in a workgroup as fit its 256 lanes, the
+// products and epilogues as in k_spmm_b1v. The dots of a column are summed
+// over the workgroup's rows through LDS, `parts` lanes a column. Bound by the
+// gathers: one row's entry is one wide load a lane, where a column per lane
+// leaves R mod 64 lanes idle and loads 4 to 16 bytes a lane. Measured (a moment
+// step, column-per-lane / slabs): 1,048,576 rows of four entries, FP64 R = 10
+// 120 / 70 us, one phase column 48 / 19; 479,596 rows of thirteen, R = 10 85 /
+// 49, R = 10 complex 141 / 108, R = 24 204 / 128; 59,212 rows of thirteen, R =
+// 10 complex 19.5 / 14.8, R = 64 51 / 31. Loading a group's indices and values
+// with wide loads changed nothing; folding the one to three last entries into
+// a masked group of four cost 10 % at thirteen entries.
+template <typename S, bool CV>
+__global__ __launch_bounds__(256) void k_spmm_b1g(int64_t nbr, int cpr, int ulen, int xcd,
+                                                  const int64_t *__restrict__ row_ptr,
+                                                  const int32_t *__restrict__ col_ind, const S *__restrict__ vals,
+                                                  const S *__restrict__ X, S *__restrict__ Y, EpiArgs e) {
+    using VT = std::conditional_t<CV, typename V2<S>::T, S>;
+    constexpr int NS = 16 / (int)sizeof(S);   // scalars a lane owns in a row
+    constexpr int CPL = NS / (CV ? 2 : 1);    // columns
+    typedef S C16 __attribute__((ext_vector_type(NS)));
+    const int rpb = 256 / cpr;
+    const int lr = (int)threadIdx.x / cpr, q = (int)threadIdx.x - lr * cpr;
+    const int64_t W = (int64_t)cpr * NS, lo = (int64_t)q * NS;
+    const int mode = e.mode;
+    const int ndot = dev_ndot(mode);
+    const S *__restrict__ XS = static_cast<const S *>(e.xs);
+    const S *__restrict__ XP = static_cast<const S *>(e.xp);
+    const S *__restrict__ PSI = static_cast<const S *>(e.psi);
+    auto ld = [](const S *p) { return *reinterpret_cast<const C16 *>(p); };
+    auto vt = [](C16 v, int j) -> VT {
+        if constexpr (CV) return VT{v[2 * j], v[2 * j + 1]};
+        else return v[j];
+    };
+    auto aff = [](C16 v, double a, double b, C16 s) -> C16 {
+        C16 o;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) o[i] = affine(v[i], a, b, s[i]);
+        return o;
+    };
+    double2 dacc[3][CPL];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int j = 0; j < CPL; ++j) dacc[d][j] = double2{0.0, 0.0};
+
+    const RowWalk walk(nbr, rpb, xcd);
+    for (int64_t base = walk.lo; base < walk.hi; base += walk.step) {
+        const int64_t br = base + lr;
+        if (lr >= rpb || br >= walk.hi) continue;
+        const int64_t s0 = ulen > 0 ? br * ulen : row_ptr[br];
+        const int64_t s1 = ulen > 0 ? s0 + ulen : row_ptr[br + 1];
+        C16 y = C16(S(0));
+        int64_t s = s0;
+        constexpr int U = 4;
+        for (; s + U <= s1; s += U) {
+            int32_t c[U];
+            S a[U];
+            C16 g[U];
+#pragma unroll
+            for (int t = 0; t < U; ++t) {
+                c[t] = col_ind[s + t];
+                a[t] = vals[s + t];
+            }
+#pragma unroll
+            for (int t = 0; t < U; ++t) g[t] = ld(X + c[t] * W + lo);
+#pragma unroll
+            for (int t = 0; t < U; ++t)
+#pragma unroll
+                for (int i = 0; i < NS; ++i) {
+                    S yi = y[i];
+                    mac(yi, a[t], (S)g[t][i]);
+                    y[i] = yi;
+                }
+        }
+        for (; s < s1; ++s) {
+            const C16 g = ld(X + (int64_t)col_ind[s] * W + lo);
+            const S a = vals[s];
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                S yi = y[i];
+                mac(yi, a, (S)g[i]);
+                y[i] = yi;
+            }
+        }
+        const int64_t idx = br * W + lo;
+        if (mode == EPI_FIRST) {
+            const C16 xs = ld(XS + idx);
+            y = aff(y, e.alpha, e.beta, xs);
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                dotacc(dacc[0][j], vt(xs, j), vt(xs, j));
+                dotacc(dacc[1][j], vt(xs, j), vt(y, j));
+                dotacc(dacc[2][j], vt(y, j), vt(y, j));
+            }
+        } else if (mode != EPI_PLAIN) {
+            const C16 xs = ld(XS + idx), xp = ld(XP + idx);
+            y = aff(y, e.alpha, e.beta, xs) - xp;
+            if (mode == EPI_STEP) {
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) {
+                    dotacc(dacc[0][j], vt(y, j), vt(y, j));
+                    dotacc(dacc[1][j], vt(y, j), vt(xs, j));
+                }
+            } else if (mode == EPI_PLAINSTEP) {
+                const C16 ps = ld(PSI + idx);
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) dotacc(dacc[0][j], vt(ps, j), vt(y, j));
+            } else {
+                y = aff(y, 1.0, e.cm, ld(static_cast<const S *>(e.qm) + idx));
+                y = aff(y, 1.0, e.cz, ld(static_cast<const S *>(e.qz) + idx));
+                y = aff(y, 1.0, e.cp, ld(static_cast<const S *>(e.qp) + idx));
+            }
+        }
+        *reinterpret_cast<C16 *>(Y + idx) = y;
+    }
+    if (ndot == 0) return;
+    const int ncol = cpr * CPL, parts = min(min(rpb, 16), max(1, 256 / ncol));
+    __shared__ double2 sm[256 * CPL], sp[256];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= ndot) break;
+        if (lr < rpb)
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) sm[lr * ncol + q * CPL + j] = dacc[d][j];
+        __syncthreads();
+        for (int t = threadIdx.x; t < ncol * parts; t += 256) {
+            const int u = t % ncol, p = t / ncol;
+            double2 v{0.0, 0.0};
+            for (int r = p; r < rpb; r += parts) {
+                v.x += sm[r * ncol + u].x;
+                v.y += sm[r * ncol + u].y;
+            }
+            if (parts == 1) e.partials[((int64_t)blockIdx.x * ndot + d) * ncol + u] = v;
+            else sp[t] = v;
+        }
+        __syncthreads();
+        if (parts > 1 && (int)threadIdx.x < ncol) {
+            double2 v = sp[threadIdx.x];
+            for (int p = 1; p < parts; ++p) {
+                v.x += sp[p * ncol + threadIdx.x].x;
+                v.y += sp[p * ncol + threadIdx.x].y;
+            }
+            e.partials[((int64_t)blockIdx.x * ndot + d) * ncol + threadIdx.x] = v;
+        }
+    }
+}
+
+int xcd_walk(const BsrDev &A, int grid, int64_t row_bytes) {
+    return g_mfma.xcd_map && grid % 8 == 0 && A.nbr * row_bytes <= kXcdVectorBytes;
+}
+
+// Lanes per row (16-byte pieces) of k_spmm_b1g for this launch shape, or 0
+// when it does not apply.
+int b1g_cpr(const BsrDev &A, bool fp32, bool cv, int R) {
+    if (A.b != 1 || A.is_complex || g_b1v_bytes == 0) return 0;
+    const int bytes = R * (fp32 ? 4 : 8) * (cv ? 2 : 1);
+    if (bytes % 16 != 0 || bytes / 16 > 256) return 0;
+    const int cpr = bytes / 16;
+    const int64_t g = (A.nbr + 256 / cpr - 1) / (256 / cpr);
+    const bool longrow = g_b1g_min_grid > 0 && A.nnzb >= kLongRow * A.nbr;
+    return g >= (longrow ? std::min(g_b1g_min_grid, kLongRowMinGrid) : g_b1g_min_grid) ? cpr : 0;
+}
+
+template <typename S, bool CV>
+hipError_t go_b1g(int cpr, const BsrDev &A, const void *X, void *Y, const EpiArgs &e, int grid, hipStream_t st) {
+    hipLaunchKernelGGL((k_spmm_b1g<S, CV>), dim3(grid), dim3(256), 0, st, A.nbr, cpr, g_uniform_rows ? A.ulen : 0,
+                       xcd_walk(A, grid, (int64_t)cpr * 16), A.row_ptr, A.col_ind, static_cast<const S *>(A.vals),
+                       static_cast<const S *>(X), static_cast<S *>(Y), e);
+    return hipGetLastError();
+}
+
 // Lanes per row of the slab layout for this launch shape, or 0 when it does
 // not apply: b = 1, real matrix, R of 16 or 32, g_b1v_bytes a lane.
 int b1v_lpr(const BsrDev &A, bool fp32, bool cv, int R) {
@@ -569,8 +775,9 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 template <typename S, bool CV, int LPR, int CPL>
 hipError_t go_b1v(const BsrDev &A, const void *X, void *Y, const EpiArgs &e, int grid, hipStream_t st) {
     hipLaunchKernelGGL((k_spmm_b1v<S, CV, LPR, CPL>), dim3(grid), dim3(64 * kWaves), 0, st, A.nbr,
-                       g_uniform_rows ? A.ulen : 0, A.row_ptr, A.col_ind, static_cast<const S *>(A.vals),
-                       static_cast<const S *>(X), static_cast<S *>(Y), e);
+                       g_uniform_rows ? A.ulen : 0, xcd_walk(A, grid, (int64_t)LPR * CPL * (CV ? 2 : 1) * sizeof(S)),
+                       A.row_ptr, A.col_ind, static_cast<const S *>(A.vals), static_cast<const S *>(X),
+                       static_cast<S *>(Y), e);
     return hipGetLastError();
 }
 
@@ -767,6 +974,17 @@ int valu_grid(int64_t nbr, int lpr) {
 }
 } // namespace
 
+// Workgroups of the VALU SpMM for this operand, by the layout the launch takes.
+static int valu_launch_grid(const BsrDev &A, VecMode vm, int R) {
+    if (b1v_lpr(A, vm.fp32, vm.complex_vec, R) == 0)
+        if (const int cpr = b1g_cpr(A, vm.fp32, vm.complex_vec, R)) {
+            const int64_t rpb = 256 / cpr, g = ((A.nbr + rpb - 1) / rpb + 7) / 8 * 8; // whole XCD rounds
+            return (int)(g > kMaxGrid ? kMaxGrid : g);
+        }
+    const int g = valu_grid(A.nbr, valu_lpr(A, vm.fp32, vm.complex_vec, R));
+    return b1v_lpr(A, vm.fp32, vm.complex_vec, R) ? (g + 7) / 8 * 8 : g;
+}
+
 int spmm_grid(int64_t nbr, int R) {
     const int G = 64 / lpr_for(R);
     const int64_t rows_per_wg = (int64_t)kWaves * G;
@@ -835,7 +1053,7 @@ int spmm_launch_grid(const BsrDev &A, VecMode vm, int R) {
         t_mfma_grid_query = false;
         return he == hipSuccess ? g : kMaxGrid;
     }
-    return valu_grid(A.nbr, valu_lpr(A, vm.fp32, vm.complex_vec, R));
+    return valu_launch_grid(A, vm, R);
 }
 
 hipError_t launch_spmm(const BsrDev &A, VecMode vm, const void *X, void *Y, int R,
@@ -851,17 +1069,23 @@ hipError_t launch_spmm(const BsrDev &A, VecMode vm, const void *X, void *Y, int 
     }
     // sized by the layout the launch takes (the wide b = 1 layout covers twice
     // the rows per workgroup)
-    const int grid = valu_grid(A.nbr, valu_lpr(A, vm.fp32, vm.complex_vec, R));
+    const int grid = valu_launch_grid(A, vm, R);
     if (grid_out) *grid_out = grid;
-    if (const int lpr = b1v_lpr(A, vm.fp32, vm.complex_vec, R)) {
-        const void *ops[] = {X, Y, e.xs, e.xp, e.psi, e.qm, e.qz, e.qp};
-        bool ok = true;
-        for (const void *o : ops) ok = ok && aligned16(o);
-        if (ok) {
+    const void *ops[] = {X, Y, e.xs, e.xp, e.psi, e.qm, e.qz, e.qp};
+    bool ok = true;
+    for (const void *o : ops) ok = ok && aligned16(o);
+    if (ok) {
+        if (const int lpr = b1v_lpr(A, vm.fp32, vm.complex_vec, R)) {
             if (vm.fp32) return vm.complex_vec ? by_b1v<float, true>(lpr, A, X, Y, R, e, grid, stream)
                                                : by_b1v<float, false>(lpr, A, X, Y, R, e, grid, stream);
             return vm.complex_vec ? by_b1v<double, true>(lpr, A, X, Y, R, e, grid, stream)
                                   : by_b1v<double, false>(lpr, A, X, Y, R, e, grid, stream);
+        }
+        if (const int cpr = b1g_cpr(A, vm.fp32, vm.complex_vec, R)) {
+            if (vm.fp32) return vm.complex_vec ? go_b1g<float, true>(cpr, A, X, Y, e, grid, stream)
+                                               : go_b1g<float, false>(cpr, A, X, Y, e, grid, stream);
+            return vm.complex_vec ? go_b1g<double, true>(cpr, A, X, Y, e, grid, stream)
+                                  : go_b1g<double, false>(cpr, A, X, Y, e, grid, stream);
         }
     }
     if (!vm.fp32) {
@@ -882,7 +1106,10 @@ void set_mfma_grid_cap(int g) { g_mfma.grid_cap = g >= 8 && g <= kMaxGrid ? (g /
 void set_b1_wide(int mode) { g_b1_wide = mode == 0 || mode == 1 ? mode : 2; }
 void set_uniform_rows(int on) { g_uniform_rows = on != 0; }
 void set_b1_slab(int bytes) { g_b1v_bytes = bytes == 0 || bytes == 16 || bytes == 32 || bytes == 64 ? bytes : -1; }
-void set_b1_slab_min_grid(int g) { g_b1v_min_grid = g >= 0 ? g : 512; }
+void set_b1_slab_min_grid(int g) {
+    g_b1v_min_grid = g >= 0 ? g : 512;
+    g_b1g_min_grid = g >= 0 ? g : 1024;
+}
 hipError_t launch_block_transpose(const double *in, double *out, int64_t nnzb, int b, bool cplx,
                                   hipStream_t stream) {
     hipLaunchKernelGGL(k_block_transpose, dim3(grid_1d(nnzb * b * b)), dim3(256), 0, stream, in,
