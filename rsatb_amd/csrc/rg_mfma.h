@@ -224,20 +224,19 @@ __device__ __forceinline__ void mfma_epilogue(const typename Acc4<S>::T (&acc)[N
     const S *__restrict__ XS = static_cast<const S *>(e.xs);
     const S *__restrict__ XP = static_cast<const S *>(e.xp);
     const S *__restrict__ PSI = static_cast<const S *>(e.psi);
-    // one output row per pass keeps the epilogue's registers low (unrolling
-    // it costs occupancy and time)
-#pragma unroll 1
+    // one output row per pass keeps the epilogue's registers low: the barrier
+    // holds the next passes' loads back. Written out: picking a pass's
+    // accumulator element in a loop took a tree of branches per tile
+#pragma unroll
     for (int v = 0; v < 4; ++v) {
+        __builtin_amdgcn_sched_barrier(0);
         // accumulator element v holds row 4 v + g (f64) or 4 g + v (f32)
         const int r = sizeof(S) == 8 ? 4 * v + g : 4 * g + v;
         if (r >= b) continue;
         const int64_t base = (br * b + r) * (int64_t)W + col0;
         S y[NT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            // element v of acc[t], selected without dynamic indexing
-            y[t] = v == 0 ? acc[t][0] : v == 1 ? acc[t][1] : v == 2 ? acc[t][2] : acc[t][3];
-        }
+        for (int t = 0; t < NT; ++t) y[t] = acc[t][v];
         // the next pass's output row of this lane (PRE loads it early)
         const int rn = sizeof(S) == 8 ? 4 * (v + 1) + g : 4 * g + v + 1;
         const bool next = PRE && v < 3 && rn < b;
@@ -370,11 +369,21 @@ template <typename S, int NT, int MODE, bool CV, bool CM> constexpr int prefetch
     if (NT == 2) return 6;
     if (NT == 4) return 4;
     if (sizeof(S) == 8) return MODE == EPI_PLAIN ? 3 : 2;
-    return NT == 16 && CV && (MODE == EPI_PLAIN || MODE == EPI_STEP) ? 2 : 3;
+    return NT == 16 && (MODE == EPI_STEP || (CV && MODE == EPI_PLAIN)) ? 2 : 3;
 }
 
+// What bounds it, at 4,096 rows of 17 blocks of 13 x 13, FP64, W = 128 (103 us;
+// parts of the kernel taken out one at a time): the MFMAs alone are 51 us (a
+// fifth of it padding 13 rows to 16), operands from L2 add 20, their misses 12,
+// and the epilogue's streams 25. Waves of a SIMD in step, a start or a priority
+// apart, deeper buffers, and fetching the next row's first steps during the
+// epilogue all left the time where it was or raised it. Two waves a SIMD as launch
+// bounds keep the accumulators in VGPRs (at sixteen FP64 tiles they need the
+// AGPRs and one wave): with the written-out epilogue and the masked row pick,
+// FP64 W = 128 107.5 -> 102.5 us plain and 109.6 -> 103.1 step; 8,000 rows, FP32
+// W = 256 216 -> 205, 236 -> 223 and 290 -> 253 us (first).
 template <typename S, int NT, int E, bool MASK, int MODE, bool CV, bool CM>
-__global__ __launch_bounds__(256) void k_spmm_mfma(int64_t nbr, int b,
+__global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spmm_mfma(int64_t nbr, int b,
                                                    const int64_t *__restrict__ row_ptr,
                                                    const int32_t *__restrict__ xrow,
                                                    const S *__restrict__ vals,
@@ -428,6 +437,7 @@ __global__ __launch_bounds__(256) void k_spmm_mfma(int64_t nbr, int b,
     }
     dacc.zero();
 
+    const int32_t m0 = g == 0 ? -1 : 0, m1 = g == 1 ? -1 : 0, m2 = g == 2 ? -1 : 0, m3 = g == 3 ? -1 : 0;
     for (int64_t it = kq * kMfmaWaves + wave; it < total; it += nk * kMfmaWaves) {
         const int64_t pos = r_lo + it / nchunks;
         const int64_t br = sched ? (int64_t)sched[pos] : pos;
@@ -462,7 +472,8 @@ __global__ __launch_bounds__(256) void k_spmm_mfma(int64_t nbr, int b,
         int64_t kb = s0 * b;
         int32_t nx0 = xrow[kb], nx1 = xrow[kb + 1], nx2 = xrow[kb + 2], nx3 = xrow[kb + 3];
         auto fetch = [&](AT &a, S (&bv)[NT]) {
-            const int64_t xr = g == 0 ? nx0 : g == 1 ? nx1 : g == 2 ? nx2 : nx3;
+            // masks, not a select: the compiler branched over the lane groups
+            const int64_t xr = (nx0 & m0) | (nx1 & m1) | (nx2 & m2) | (nx3 & m3);
             const int k = 4 * fst + g;
             a = __builtin_nontemporal_load((i < b && k < K) ? panel + (int64_t)k * b + i
                                                             : reinterpret_cast<const AT *>(zero));
