@@ -175,7 +175,7 @@ struct rg_context {
     DevBuf sk_ints, sk_dbls, sk_type, sk_pos, sk_ei, sk_sh, sk_eblk, sk_flags, sk_sp, sk_src, sk_ph, sk_row;
     DevBuf den_in, den_out; // density reconstruction: weights and grid, result
     // Kubo-Greenwood: stored left/right sequences and the moment matrices
-    DevBuf kg_store, kg_mu, kg_work;
+    DevBuf kg_store, kg_mu, kg_work, kg_part;
     size_t kg_widen_bytes = (size_t)8 << 30; // FP32 transport: FP64 chunk panels (RG_KG_WIDEN_BYTES)
     rocblas_handle blas = nullptr;
 
@@ -2074,14 +2074,17 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     const size_t eb = vec_elem_bytes(vm), K = (size_t)rows * R, nb = K * eb;
     for (int i = 0; i < 3; ++i) RG_HIP(ctx, ctx->vec[i].ensure(nb), "hipMalloc work vector");
     RG_HIP(ctx, ctx->partials.ensure((size_t)spmm_max_grid() * 3 * R * 16), "hipMalloc partials");
-    // [left | right | left tangent | right tangent][axis][moment] vectors of K elements
-    RG_HIP(ctx, ctx->kg_store.ensure((tangent ? 12 : 6) * (size_t)M * nb), "hipMalloc sequence store");
+    // [left | right | left tangent | right tangent][axis][moment] vectors of K
+    // elements, an odd multiple of 256 bytes apart: the moment products read one
+    // place of many vectors at once, which a power of two puts on one channel
+    const size_t vb = ((nb + 255) / 256 | 1) * 256, Kp = vb / eb;
+    RG_HIP(ctx, ctx->kg_store.ensure((tangent ? 12 : 6) * (size_t)M * vb), "hipMalloc sequence store");
     if (tangent) RG_HIP(ctx, ctx->kg_work.ensure(4 * nb), "hipMalloc tangent work vectors");
     char *store = static_cast<char *>(ctx->kg_store.p);
-    auto Lst = [&](int a, int m) { return (void *)(store + ((size_t)a * M + m) * nb); };
-    auto Rst = [&](int a, int m) { return (void *)(store + ((size_t)(3 + a) * M + m) * nb); };
-    auto Ldt = [&](int a, int m) { return (void *)(store + ((size_t)(6 + a) * M + m) * nb); };
-    auto Rdt = [&](int a, int m) { return (void *)(store + ((size_t)(9 + a) * M + m) * nb); };
+    auto Lst = [&](int a, int m) { return (void *)(store + ((size_t)a * M + m) * vb); };
+    auto Rst = [&](int a, int m) { return (void *)(store + ((size_t)(3 + a) * M + m) * vb); };
+    auto Ldt = [&](int a, int m) { return (void *)(store + ((size_t)(6 + a) * M + m) * vb); };
+    auto Rdt = [&](int a, int m) { return (void *)(store + ((size_t)(9 + a) * M + m) * vb); };
     const int64_t nvec = (int64_t)K * (vm.complex_vec ? 2 : 1); // doubles per vector
 
     const double ha = ctx->half_width, c = ctx->center;
@@ -2110,7 +2113,7 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
         const BsrDev Hd = dev_view(H, fp32);
         km.h = Hd.vals;
         for (int a = 0; a < 3; ++a) km.b[a] = dev_view(ctx->slots[RG_SLOT_VX + a], fp32).vals;
-        km.left_stride = km.right_stride = (int64_t)M * nvec;
+        km.left_stride = km.right_stride = (int64_t)(M * Kp) * (vm.complex_vec ? 2 : 1);
         km.alpha1 = first.alpha;
         km.beta1 = first.beta;
         km.alpha = step.alpha;
@@ -2278,57 +2281,24 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     double *Qz = Wz + 3 * zmat;
     double *dmud = Qz + 3 * (size_t)np * zmat; // tangent moments (mu_real doubles)
     const double s2 = 1.0 / (4.0 * ha * ha);
-    // out[pi] (+)= s^2 Lseq(a)^H Rseq(b) for every pair
-    // FP32 sequences: K is cut into chunks of Kc rows; each chunk of the M
+    // out[pi] (+)= s^2 Lseq(a)^H Rseq(b) for every pair: real sequences in one
+    // launch (k_kg_gemm), complex ones a library product each.
+    // Complex FP32 sequences: K is cut into chunks of Kc rows; each chunk of the M
     // left and M right vectors is widened to FP64 (k_widen_cols) and the
     // GEMMs accumulate over the chunks in FP64 (beta = 1 after the first).
     // Chunks stay long (8 GiB of panels by default): an M x M product over a
     // short K has too few output tiles to fill the GPU (1 GiB chunks at M =
     // 512 made the FP32 spectrum 5x slower than FP64).
-    const int cw = vm.complex_vec ? 2 : 1; // floats per element
+    const int cw = 2; // floats per element
     size_t Kc = K;
-    if (fp32) {
+    if (fp32 && vm.complex_vec) {
         const size_t budget = ctx->kg_widen_bytes; // bytes of the two FP64 chunk panels
         Kc = std::max<size_t>(1, std::min(K, budget / (2 * (size_t)M * 8 * cw)));
         RG_HIP(ctx, ctx->kg_work.ensure(2 * (size_t)M * Kc * 8 * cw), "hipMalloc widening panels");
     }
-    auto moment_gemms = [&](auto Lseq, auto Rseq, double *out, double beta_in) -> int {
-    if (fp32) {
-        double *Lw = static_cast<double *>(ctx->kg_work.p);
-        double *Rw = Lw + (size_t)M * Kc * cw;
-        for (int pi = 0; pi < np; ++pi) {
-            const int a = comp_a[pairs[pi]], b = comp_b[pairs[pi]];
-            for (size_t k0 = 0; k0 < K; k0 += Kc) {
-                const size_t kc = std::min(Kc, K - k0);
-                RG_HIP(ctx, launch_widen_cols(static_cast<const float *>(Lseq(a, 0)) + k0 * cw, (int64_t)K * cw,
-                                              Lw, (int64_t)kc * cw, M, ctx->stream),
-                       "widen launch");
-                RG_HIP(ctx, launch_widen_cols(static_cast<const float *>(Rseq(b, 0)) + k0 * cw, (int64_t)K * cw,
-                                              Rw, (int64_t)kc * cw, M, ctx->stream),
-                       "widen launch");
-                const double bk = k0 == 0 ? beta_in : 1.0;
-                rocblas_status st;
-                if (vm.complex_vec) {
-                    const rocblas_double_complex alpha{s2, 0.0}, beta{bk, 0.0};
-                    st = rocblas_zgemm(ctx->blas, rocblas_operation_conjugate_transpose, rocblas_operation_none, M,
-                                       M, (rocblas_int)kc, &alpha, reinterpret_cast<rocblas_double_complex *>(Lw),
-                                       (rocblas_int)kc, reinterpret_cast<rocblas_double_complex *>(Rw),
-                                       (rocblas_int)kc, &beta,
-                                       reinterpret_cast<rocblas_double_complex *>(out + pi * zmat), M);
-                } else {
-                    const double alpha = s2;
-                    st = rocblas_dgemm(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, M, M,
-                                       (rocblas_int)kc, &alpha, Lw, (rocblas_int)kc, Rw, (rocblas_int)kc, &bk,
-                                       out + pi * mm, M);
-                }
-                if (st != rocblas_status_success) return fail(ctx, RG_ERR_HIP, "moment GEMM failed");
-            }
-        }
-        return RG_OK;
-    }
-    for (int pi = 0; pi < np; ++pi) {
-        const int a = comp_a[pairs[pi]], b = comp_b[pairs[pi]];
-        rocblas_status st;
+    const KgGemmPlan gp = kg_gemm_plan(M, (int64_t)K);
+    if (!vm.complex_vec) RG_HIP(ctx, ctx->kg_part.ensure(kg_gemm_bytes(gp, np)), "hipMalloc moment parts");
+    auto timed = [&](int products, auto run) -> int { // run() as one launch of the product class
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
         if (ctx->prof) {
             ev0 = take_event(ctx);
@@ -2336,30 +2306,62 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
             if (!ev0 || !ev1) return fail(ctx, RG_ERR_HIP, "hipEventCreate failed");
             RG_HIP(ctx, hipEventRecord(ev0, ctx->stream), "hipEventRecord");
         }
-        if (vm.complex_vec) {
-            const rocblas_double_complex alpha{s2, 0.0}, beta{beta_in, 0.0};
-            st = rocblas_zgemm(ctx->blas, rocblas_operation_conjugate_transpose, rocblas_operation_none, M, M,
-                               (rocblas_int)K, &alpha, static_cast<const rocblas_double_complex *>(Lseq(a, 0)),
-                               (rocblas_int)K, static_cast<const rocblas_double_complex *>(Rseq(b, 0)),
-                               (rocblas_int)K, &beta, reinterpret_cast<rocblas_double_complex *>(out + pi * zmat),
-                               M);
-        } else {
-            const double alpha = s2, beta = beta_in;
-            st = rocblas_dgemm(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, M, M, (rocblas_int)K,
-                               &alpha, static_cast<const double *>(Lseq(a, 0)), (rocblas_int)K,
-                               static_cast<const double *>(Rseq(b, 0)), (rocblas_int)K, &beta, out + pi * mm, M);
+        const int rr = run();
+        if (rr || !ctx->prof) return rr;
+        RG_HIP(ctx, hipEventRecord(ev1, ctx->stream), "hipEventRecord");
+        ctx->pending.push_back({ev0, ev1, RG_KCLASS_KG_GEMM});
+        // algorithmic: both sequence blocks read once, mu written once
+        const double cplx = vm.complex_vec ? 2.0 : 1.0;
+        ctx->stats[RG_KCLASS_KG_GEMM].bytes = products * (2.0 * (double)M * (double)K * eb + (double)mm * 8 * cplx);
+        ctx->stats[RG_KCLASS_KG_GEMM].flops =
+            products * 2.0 * (double)mm * (double)K * (vm.complex_vec ? 4.0 : 1.0);
+        return RG_OK;
+    };
+    auto zgemm = [&](const void *L, const void *R_, size_t kn, size_t ld, double bk, double *o) -> int {
+        const rocblas_double_complex alpha{s2, 0.0}, beta{bk, 0.0};
+        return rocblas_zgemm(ctx->blas, rocblas_operation_conjugate_transpose, rocblas_operation_none, M, M,
+                             (rocblas_int)kn, &alpha, static_cast<const rocblas_double_complex *>(L), (rocblas_int)ld,
+                             static_cast<const rocblas_double_complex *>(R_), (rocblas_int)ld, &beta,
+                             reinterpret_cast<rocblas_double_complex *>(o), M) == rocblas_status_success
+                   ? RG_OK
+                   : fail(ctx, RG_ERR_HIP, "moment GEMM failed");
+    };
+    auto moment_gemms = [&](auto Lseq, auto Rseq, double *out, double beta_in) -> int {
+        if (!vm.complex_vec) {
+            KgGemm p{};
+            for (int pi = 0; pi < np; ++pi) {
+                p.l[pi] = Lseq(comp_a[pairs[pi]], 0);
+                p.r[pi] = Rseq(comp_b[pairs[pi]], 0);
+            }
+            return timed(np, [&]() -> int {
+                RG_HIP(ctx, launch_kg_gemm(gp, p, np, fp32, (int64_t)K, (int64_t)Kp, M, s2, beta_in,
+                                           static_cast<double *>(ctx->kg_part.p), out, (int64_t)mm, ctx->stream),
+                       "moment products");
+                return RG_OK;
+            });
         }
-        if (st != rocblas_status_success) return fail(ctx, RG_ERR_HIP, "moment GEMM failed");
-        if (ctx->prof) {
-            RG_HIP(ctx, hipEventRecord(ev1, ctx->stream), "hipEventRecord");
-            ctx->pending.push_back({ev0, ev1, RG_KCLASS_KG_GEMM});
-            // algorithmic: both sequence blocks read once, mu written once
-            const double cplx = vm.complex_vec ? 2.0 : 1.0;
-            ctx->stats[RG_KCLASS_KG_GEMM].bytes = 2.0 * (double)M * (double)K * eb + (double)mm * 8 * cplx;
-            ctx->stats[RG_KCLASS_KG_GEMM].flops = 2.0 * (double)mm * (double)K * (vm.complex_vec ? 4.0 : 1.0);
+        for (int pi = 0; pi < np; ++pi) {
+            const int a = comp_a[pairs[pi]], b = comp_b[pairs[pi]];
+            if (!fp32) {
+                const int rr = timed(1, [&]() { return zgemm(Lseq(a, 0), Rseq(b, 0), K, Kp, beta_in, out + pi * zmat); });
+                if (rr) return rr;
+                continue;
+            }
+            double *Lw = static_cast<double *>(ctx->kg_work.p);
+            double *Rw = Lw + (size_t)M * Kc * cw;
+            for (size_t k0 = 0; k0 < K; k0 += Kc) {
+                const size_t kc = std::min(Kc, K - k0);
+                RG_HIP(ctx, launch_widen_cols(static_cast<const float *>(Lseq(a, 0)) + k0 * cw, (int64_t)Kp * cw,
+                                              Lw, (int64_t)kc * cw, M, ctx->stream),
+                       "widen launch");
+                RG_HIP(ctx, launch_widen_cols(static_cast<const float *>(Rseq(b, 0)) + k0 * cw, (int64_t)Kp * cw,
+                                              Rw, (int64_t)kc * cw, M, ctx->stream),
+                       "widen launch");
+                const int rr = zgemm(Lw, Rw, kc, kc, k0 == 0 ? beta_in : 1.0, out + pi * zmat);
+                if (rr) return rr;
+            }
         }
-    }
-    return RG_OK;
+        return RG_OK;
     };
     rc = moment_gemms(Lst, Rst, mud, 0.0);
     if (!rc && tangent) rc = moment_gemms(Ldt, Rst, dmud, 0.0);

@@ -13,6 +13,7 @@
 // launches 7.5 us each, 52 us a moment; 23 us a moment here (126 MB, 5.5 TB/s).
 #include "rg_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rg {
@@ -127,6 +128,133 @@ __global__ __launch_bounds__(256) void k_kg_moment(int64_t n, int ulen, const in
     if (a.y) put(a.y, recur(y, a.x, a.xp));
 }
 
+// ------------------------------------------------------- moment products
+// mu^{ab} = alpha L_a^T R_b of real sequences: M x M outputs over K = rows R,
+// each sequence M vectors of K contiguous elements. The chip is filled by cutting
+// K: a workgroup of 2 x 2 waves owns a T x T tile (T = 32 A) of one chunk of K,
+// and k_kg_sum adds the chunks in order. A lane of an MFMA operand takes four
+// K elements in 16-byte accesses, so a row's four lane groups load 64 contiguous
+// bytes each time (FP32 is widened in registers: products of two FP32 values
+// are exact), and four MFMAs take one element each; no LDS. Rows lie ld
+// apart and have at least sixteen elements of memory. The tiles of a chunk run on
+// one XCD, whose L2 holds the chunk's rows. Bound by the MFMAs (M^2 K / 36.6
+// TF/s) above M of about 100, by reading the sequences below.
+// Measured, three products, against rocBLAS, which cuts K only for some sizes:
+// M = 256, K = 1,048,576 7.5 -> 7.0 ms; M = 200 7.0 -> 7.5; M = 90, K = 409,600
+// 2.35 -> 0.47; M = 128, K = 120,000 58 -> 0.22; M = 512, K = 131,072 63 -> 3.5;
+// M = 1024, K = 73,728 36 -> 14; M = 64, K = 4,096 0.67 -> 0.01. Vectors a power of
+// two apart took 10.6 instead of 9.6 ms, a masked tail of scalar loads in the
+// loop 9.6 instead of 7.0. Error of the moments against 80-bit sums (rel. 2-norm),
+// library / here: K = 36,000, M = 128 5.1e-15 / 2.9e-16; K = 96,000, M = 96
+// 8.7e-15 / 2.0e-16: shorter chains of additions.
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+template <typename S, int A>
+__global__ __launch_bounds__(256, 1) void k_kg_gemm(KgGemm p, int64_t K, int64_t ld, int64_t kc, int M, int nt, int nchunk,
+                                                    double *__restrict__ part) {
+    constexpr int T = 32 * A;
+    constexpr int E = 16 / (int)sizeof(S), P = 4 / E; // elements of an access, accesses a row
+    typedef S SE __attribute__((ext_vector_type(E), aligned(sizeof(S))));
+    const int tiles = nt * nt, rest = (int)blockIdx.x >> 3;
+    const int tile = rest % tiles, chunk = (rest / tiles) * 8 + ((int)blockIdx.x & 7);
+    if (chunk >= nchunk) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i = lane & 15, g = lane >> 4;
+    const int m0 = (tile / nt) * T + (wave >> 1) * 16 * A, n0 = (tile % nt) * T + (wave & 1) * 16 * A;
+    const S *__restrict__ lp[A], *__restrict__ rp[A];
+#pragma unroll
+    for (int r = 0; r < A; ++r) { // rows past M load the last one and are not stored
+        lp[r] = static_cast<const S *>(p.l[blockIdx.y]) + (int64_t)min(m0 + 16 * r + i, M - 1) * ld;
+        rp[r] = static_cast<const S *>(p.r[blockIdx.y]) + (int64_t)min(n0 + 16 * r + i, M - 1) * ld;
+    }
+    const int64_t k0 = chunk * kc, k1 = min(K, k0 + kc);
+    d4 acc[A][A];
+#pragma unroll
+    for (int r = 0; r < A; ++r)
+#pragma unroll
+        for (int c = 0; c < A; ++c) acc[r][c] = d4(0.0);
+    // The last block of K starts at klast: a ragged one repeats elements, which
+    // are zeroed when it is used (as is what lies past a K below 16).
+    const int64_t klast = max(K - 16, (int64_t)0);
+    auto load = [&](int64_t k, d4 (&a)[A], d4 (&b)[A]) {
+        const int64_t kk = min(k, klast) + E * g;
+#pragma unroll
+        for (int r = 0; r < A; ++r)
+#pragma unroll
+            for (int q = 0; q < P; ++q) {
+                const SE x = *reinterpret_cast<const SE *>(lp[r] + kk + 4 * E * q);
+                const SE y = *reinterpret_cast<const SE *>(rp[r] + kk + 4 * E * q);
+#pragma unroll
+                for (int j = 0; j < E; ++j) {
+                    a[r][E * q + j] = (double)x[j];
+                    b[r][E * q + j] = (double)y[j];
+                }
+            }
+    };
+    d4 a0[A], b0[A], a1[A], b1[A];
+    load(k0, a0, b0);
+    for (int64_t k = k0; k < k1; k += 16) {
+        load(k + 16 < k1 ? k + 16 : k0, a1, b1);
+        __builtin_amdgcn_sched_barrier(0); // in flight during the products
+        if (k > klast || K < 16) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t e = min(k, klast) + E * g + 4 * E * (j / E) + j % E;
+                if (e < k || e >= K) {
+#pragma unroll
+                    for (int r = 0; r < A; ++r) a0[r][j] = b0[r][j] = 0.0;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < A; ++r)
+#pragma unroll
+                for (int c = 0; c < A; ++c)
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[r][j], b0[c][j], acc[r][c], 0, 0, 0);
+        // moved, not taken in turn: unrolling by two moved the accumulators
+        // between the register files on each turn (7.0 -> 7.5 ms)
+#pragma unroll
+        for (int r = 0; r < A; ++r) {
+            a0[r] = a1[r];
+            b0[r] = b1[r];
+        }
+    }
+    const int64_t Mp = (int64_t)nt * T;
+    double *__restrict__ out = part + ((int64_t)blockIdx.y * nchunk + chunk) * Mp * Mp;
+#pragma unroll
+    for (int r = 0; r < A; ++r)
+#pragma unroll
+        for (int c = 0; c < A; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) out[(int64_t)(m0 + 16 * r + 4 * v + g) * Mp + n0 + 16 * c + i] = acc[r][c][v];
+}
+
+// out[m + n M] = alpha sum over the chunks of part[m][n] + beta out[m + n M]:
+// 64 elements a workgroup, four threads each taking every fourth chunk.
+__global__ __launch_bounds__(256) void k_kg_sum(const double *__restrict__ part, int nchunk, int Mp, int M,
+                                                double alpha, double beta, double *__restrict__ out,
+                                                int64_t out_stride) {
+    __shared__ double sm[4][64];
+    const int u = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t e = (int64_t)blockIdx.x * 64 + u, mat = (int64_t)Mp * Mp;
+    const int m = (int)(e / M), n = (int)(e - (int64_t)m * M);
+    double s = 0.0;
+    if (m < M) {
+        const double *q = part + (int64_t)blockIdx.y * nchunk * mat + (int64_t)m * Mp + n;
+#pragma unroll 8
+        for (int c = w; c < nchunk; c += 4) s += q[c * mat];
+    }
+    sm[w][u] = s;
+    __syncthreads();
+    if (w == 0 && m < M) {
+        double *o = out + blockIdx.y * out_stride + (int64_t)n * M + m;
+        const double v = alpha * (sm[0][u] + sm[1][u] + sm[2][u] + sm[3][u]);
+        *o = beta == 0.0 ? v : v + beta * *o;
+    }
+}
+
 // *flag = 1 unless the two patterns are the same (their row counts are)
 __global__ __launch_bounds__(256) void k_same_pattern(int64_t n, int64_t nnz, const int64_t *__restrict__ rp,
                                                       const int64_t *__restrict__ rq, const int32_t *__restrict__ cp,
@@ -220,6 +348,49 @@ hipError_t launch_kg_moment(const BsrDev &H, VecMode vm, const KgMoment &a, int 
 hipError_t launch_same_pattern(const BsrDev &A, const BsrDev &B, int *flag, hipStream_t st) {
     hipLaunchKernelGGL(k_same_pattern, dim3(grid_for(A.nnzb + A.nbr + 1)), dim3(256), 0, st, A.nbr, A.nnzb, A.row_ptr,
                        B.row_ptr, A.col_ind, B.col_ind, flag);
+    return hipGetLastError();
+}
+
+// Tile side: the fewest padded outputs, wider on a tie; chunks of K: one
+// workgroup a CU, at least 64 elements each.
+KgGemmPlan kg_gemm_plan(int M, int64_t K) {
+    KgGemmPlan p;
+    int64_t best = 0;
+    for (int a = 4; a >= 2; --a) {
+        const int64_t side = (M + 32 * a - 1) / (32 * a) * (32 * a);
+        if (best == 0 || side < best) {
+            best = side;
+            p.a = a;
+        }
+    }
+    p.nt = (int)(best / (32 * p.a));
+    const int64_t tiles = (int64_t)p.nt * p.nt;
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>((p.a == 4 ? 256 : 512) / tiles, (K + 63) / 64));
+    p.kc = ((K + want - 1) / want + 15) / 16 * 16;
+    p.nchunk = (int)((K + p.kc - 1) / p.kc);
+    return p;
+}
+
+hipError_t launch_kg_gemm(const KgGemmPlan &pl, const KgGemm &p, int npairs, bool fp32, int64_t K, int64_t ld, int M,
+                          double alpha, double beta, double *part, double *out, int64_t out_stride, hipStream_t st) {
+    const int Mp = pl.nt * 32 * pl.a;
+    const dim3 grid((unsigned)((pl.nchunk + 7) / 8 * 8 * pl.nt * pl.nt), (unsigned)npairs);
+#define RG_KG_CASE(S_, A_)                                                                                          \
+    hipLaunchKernelGGL((k_kg_gemm<S_, A_>), grid, dim3(256), 0, st, p, K, ld, pl.kc, M, pl.nt, pl.nchunk, part)
+    if (fp32) {
+        if (pl.a == 2) RG_KG_CASE(float, 2);
+        else if (pl.a == 3) RG_KG_CASE(float, 3);
+        else RG_KG_CASE(float, 4);
+    } else {
+        if (pl.a == 2) RG_KG_CASE(double, 2);
+        else if (pl.a == 3) RG_KG_CASE(double, 3);
+        else RG_KG_CASE(double, 4);
+    }
+#undef RG_KG_CASE
+    hipError_t he = hipGetLastError();
+    if (he != hipSuccess) return he;
+    hipLaunchKernelGGL(k_kg_sum, dim3((unsigned)(((int64_t)M * M + 63) / 64), (unsigned)npairs), dim3(256), 0, st, part,
+                       pl.nchunk, Mp, M, alpha, beta, out, out_stride);
     return hipGetLastError();
 }
 
