@@ -2534,33 +2534,16 @@ int rg_isqrt_patches(rg_context *ctx, double tol, int maxit, int *iters_out, dou
     if (ld > 512)
         return fail(ctx, RG_ERR_UNSUPPORTED,
                     "patch dimension " + std::to_string(n) + " exceeds the 512 the kernel supports");
-    DevBuf buf[5], cs, resid, iters;
-    // Symmetric overlaps (to rounding) take the one-workgroup kernel; one that
-    // is not, and patches past its dimension, the general batched products.
-    bool sym = !small && n <= ns_patch_max();
-    if (sym) {
-        int flag = 0;
-        RG_HIP(ctx, iters.ensure(4), "hipMalloc");
-        RG_HIP(ctx, hipMemcpyAsync(iters.p, &flag, 4, hipMemcpyHostToDevice, ctx->stream), "clear flag");
-        RG_HIP(ctx, launch_asymmetric(nbr, b, (const int64_t *)S.row_ptr.p, (const int32_t *)S.col_ind.p,
-                                      (const double *)S.vals64.p, (int *)iters.p, ctx->stream),
-               "symmetry check");
-        RG_HIP(ctx, hipMemcpyAsync(&flag, iters.p, 4, hipMemcpyDeviceToHost, ctx->stream), "download flag");
-        RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "sync");
-        sym = flag == 0;
-    }
-    const bool whole = small || sym; // every patch in one launch
     const size_t mat = (size_t)ld * ld;
     const size_t budget = (size_t)6 << 30;
-    int64_t batch = whole ? nbr : (int64_t)std::max<size_t>(1, budget / (5 * mat * 8));
+    int64_t batch = small ? nbr : (int64_t)std::max<size_t>(1, budget / (5 * mat * 8));
     batch = std::min<int64_t>(batch, nbr);
-    const int ld16 = (n + 15) / 16 * 16, sym_grid = sym ? ns_patch_grid(nbr) : 0;
-    if (sym) RG_HIP(ctx, buf[0].ensure(ns_patch_bytes(sym_grid, ld16)), "hipMalloc patches");
-    if (!whole)
+    DevBuf buf[5], cs, resid, iters;
+    if (!small)
         for (auto &bb : buf) RG_HIP(ctx, bb.ensure((size_t)batch * mat * 8), "hipMalloc patches");
     RG_HIP(ctx, cs.ensure((size_t)batch * 8), "hipMalloc");
     RG_HIP(ctx, resid.ensure((size_t)batch * 8), "hipMalloc");
-    if (whole) RG_HIP(ctx, iters.ensure((size_t)batch * 4), "hipMalloc");
+    if (small) RG_HIP(ctx, iters.ensure((size_t)batch * 4), "hipMalloc");
     // the factor shares S's pattern
     Slot &Z = ctx->slots[RG_SLOT_Z];
     Slot &ZH = ctx->slots[RG_SLOT_ZH];
@@ -2587,15 +2570,9 @@ int rg_isqrt_patches(rg_context *ctx, double tol, int maxit, int *iters_out, dou
     int it_max = 0;
     double res_max = 0.0;
     std::vector<double> hres((size_t)batch);
-    if (whole) {
+    if (small) {
         // every patch in one launch, each iterating to its own convergence
-        if (sym)
-            RG_HIP(ctx, launch_ns_patch(nbr, sym_grid, b, (const int64_t *)S.row_ptr.p, (const int32_t *)S.col_ind.p,
-                                        (const double *)S.vals64.p, ld16, tol, maxit, (double *)buf[0].p,
-                                        (double *)Z.vals64.p, (int *)iters.p, (double *)resid.p, ctx->stream),
-                   "patch iteration");
-        else
-            RG_HIP(ctx, launch_ns_small(0, nbr, b, (const int64_t *)S.row_ptr.p, (const int32_t *)S.col_ind.p,
+        RG_HIP(ctx, launch_ns_small(0, nbr, b, (const int64_t *)S.row_ptr.p, (const int32_t *)S.col_ind.p,
                                     (const double *)S.vals64.p, tol, maxit, (double *)Z.vals64.p, (double *)cs.p,
                                     (int *)iters.p, (double *)resid.p, ctx->stream),
                "small patch iteration");
@@ -2619,7 +2596,7 @@ int rg_isqrt_patches(rg_context *ctx, double tol, int maxit, int *iters_out, dou
             res_max = std::max(res_max, r);
         }
     }
-    for (int64_t first = 0; first < (whole ? 0 : nbr); first += batch) {
+    for (int64_t first = 0; first < (small ? 0 : nbr); first += batch) {
         const int64_t cnt = std::min<int64_t>(batch, nbr - first);
         double *Y = (double *)buf[0].p, *Zm = (double *)buf[1].p, *T = (double *)buf[2].p;
         double *Y2 = (double *)buf[3].p, *Z2 = (double *)buf[4].p;

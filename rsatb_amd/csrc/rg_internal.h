@@ -201,19 +201,6 @@ hipError_t launch_density(const double *w, int64_t G, int M, const double *x, in
 hipError_t launch_patch_gather(int64_t first, int64_t count, int b, const int64_t *row_ptr,
                                const int32_t *col_ind, const double *vals, int ld, double *Y,
                                double *Z, double *cs, hipStream_t st);
-// *flag = 1 when S is not symmetric to rounding (its pattern included)
-hipError_t launch_asymmetric(int64_t nbr, int b, const int64_t *row_ptr, const int32_t *col_ind, const double *vals,
-                             int *flag, hipStream_t st);
-// symmetric patches of dimension up to ns_patch_max() (256): the whole
-// iteration per patch in one launch of ns_patch_grid() workgroups on
-// ns_patch_bytes(grid, ld) of work (ld: the largest dimension rounded up to
-// 16); the factor's block rows into zout, iters / resid per patch
-int ns_patch_max();
-int ns_patch_grid(int64_t npatch);
-size_t ns_patch_bytes(int grid, int ld);
-hipError_t launch_ns_patch(int64_t npatch, int grid, int b, const int64_t *row_ptr, const int32_t *col_ind,
-                           const double *vals, int ld, double tol, int maxit, double *work, double *zout, int *iters,
-                           double *resid, hipStream_t st);
 // mode 0: C = 1.5 I - 0.5 A B and resid[p] += ||I - A B||_F^2; mode 1: C = A B
 hipError_t launch_ns_gemm(int mode, int64_t count, int ld, const double *A, const double *B,
                           double *C, double *resid, hipStream_t st);

@@ -17,18 +17,10 @@
 // with 64 x 16 / 16 x 64 operand panels staged in LDS.
 #include "rg_internal.h"
 
-#include <type_traits>
-
 namespace rg {
 namespace {
 
 typedef double D4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
-}
 
 // block (r, c) of a BSR with sorted columns: its index, or -1
 __device__ __forceinline__ int64_t find_block(const int64_t *__restrict__ row_ptr,
@@ -197,333 +189,6 @@ __global__ __launch_bounds__(256) void k_ns_gemm(int ld, const double *__restric
     }
 }
 
-// ---- symmetric patches of dimension 17 .. 256: one workgroup per patch
-//
-// An overlap is symmetric, and with it Y, Z and T, which commute: every product
-// of the iteration is symmetric, so only the 16 x 16 tiles of its lower
-// triangle are formed, and written twice. Both operands are read as rows
-// (A[r][k] = A[k][r]).
-//
-// The batched 64 x 64-tile products (k_ns_gemm) are bound by traffic: each
-// reads its panels again for every tile, 6.4 TB/s from the fabric while the
-// MFMA pipes are half idle. Here one workgroup of sixteen waves holds a whole
-// product in its accumulators (at most nine tiles a wave), so each operand is
-// read once per product, a product may overwrite its operand, and the
-// workgroup carries its patch through all iterations on three matrices, of
-// which only the lower triangle's tiles are stored (each 16 x 16 row-major,
-// 2 KB): what 256 workgroups touch stays in the Infinity Cache (154 MB at n16 =
-// 224; with whole matrices, 308 MB, the factor below took 12.2 ms). No iteration
-// waits for the host or for another patch. Chunks of 16 k of both operands are
-// staged in LDS (a tile below the diagonal transposed on the way), the next
-// chunk's loads in flight during a chunk's MFMAs. Bound: the FP64 MFMA rate.
-// Measured at 13-orbital diamond with vacancies (1,596 patches, n <= 221), the
-// whole factor: 23.2 ms with the batched products, 10.0 ms here; 4,096 patches
-// of n = 221 57 -> 23.6 ms (60 us a product and workgroup, of which the MFMAs of
-// its tiles are 44).
-
-// 1 in *flag when a stored value of S differs from its transpose's by more
-// than rounding (8 ulp of the two diagonal entries) or has no transpose.
-__global__ __launch_bounds__(256) void k_asymmetric(int64_t nbr, int b, const int64_t *__restrict__ row_ptr,
-                                                    const int32_t *__restrict__ col_ind,
-                                                    const double *__restrict__ vals, int *__restrict__ flag) {
-    const int per = b * b;
-    for (int64_t i = blockIdx.x; i < nbr; i += gridDim.x) {
-        const int64_t s0 = row_ptr[i], n = (row_ptr[i + 1] - s0) * per;
-        const int64_t di = find_block(row_ptr, col_ind, i, (int32_t)i);
-        for (int64_t t = threadIdx.x; t < n; t += blockDim.x) {
-            const int64_t s = s0 + t / per;
-            const int e = (int)(t % per), cc = e / b, rr = e - cc * b;
-            const int32_t j = col_ind[s];
-            const int64_t s2 = find_block(row_ptr, col_ind, j, (int32_t)i), dj = find_block(row_ptr, col_ind, j, j);
-            bool ok = s2 >= 0 && di >= 0 && dj >= 0;
-            if (ok) {
-                const double tol = 1.8e-15 * (fabs(vals[di * per + rr * (b + 1)]) + fabs(vals[dj * per + cc * (b + 1)]));
-                ok = fabs(vals[s * per + e] - vals[s2 * per + rr * b + cc]) <= tol; // false for NaN
-            }
-            if (!ok) *flag = 1;
-        }
-    }
-}
-
-constexpr int kPatchMax = 256;  // largest dimension
-constexpr int kPatchTab = 64;   // block table side: patches of more blocks search per entry
-// LDS row stride: rows k and k + 1 in different bank halves (2176 = 128 mod 256
-// bytes); one for all dimensions, so that the k offsets are immediates.
-constexpr int kPatchLds = 272;
-
-// NQ: the most tiles a wave takes, at least the largest patch's ntile / 16.
-// work: three matrices of ldt tiles per workgroup. iters[p], resid[p] =
-// ||I - Z Y||_F when patch p stopped (converged below tol, diverged past 100 or
-// not finite, or maxit updates); a converged patch's rows of block i of
-// T Z / sqrt(c) go to zout (the update that its last T already stands for).
-template <int NQ>
-__global__ __launch_bounds__(1024) void k_ns_patch(int64_t npatch, int b, const int64_t *__restrict__ row_ptr,
-                                                   const int32_t *__restrict__ col_ind,
-                                                   const double *__restrict__ vals, int ldt, double tol, int maxit,
-                                                   double *work, double *__restrict__ zout, int *__restrict__ iters,
-                                                   double *__restrict__ resid) {
-    __shared__ double sm[2 * 2 * 16 * kPatchLds];
-    __shared__ double red[16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = lane & 15, g = lane >> 4;
-    double *Y = work + (int64_t)blockIdx.x * 3 * ldt * 256, *Z = Y + (int64_t)ldt * 256, *T = Z + (int64_t)ldt * 256;
-
-    // tile t of the lower triangle: its row tr (its column: t - tr (tr + 1) / 2)
-    auto tile_row = [](int t) -> int {
-        int tr = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
-        while ((tr + 1) * (tr + 2) / 2 <= t) ++tr;
-        while (tr * (tr + 1) / 2 > t) --tr;
-        return tr;
-    };
-    // entry (r, c) of a stored symmetric matrix
-    auto at = [](const double *M, int r, int c) -> double {
-        const int tr = r >> 4, tc = c >> 4;
-        return tr >= tc ? M[(tr * (tr + 1) / 2 + tc) * 256 + (r & 15) * 16 + (c & 15)]
-                        : M[(tc * (tc + 1) / 2 + tr) * 256 + (c & 15) * 16 + (r & 15)];
-    };
-
-    // the sum (or maximum) of one value per wave, in wave order
-    auto combine = [&](double v, bool max_) -> double {
-        __syncthreads();
-        if (lane == 0) red[wave] = v;
-        __syncthreads();
-        double s = red[0];
-        for (int q = 1; q < 16; ++q) s = max_ ? fmax(s, red[q]) : s + red[q];
-        return s;
-    };
-
-    for (int64_t p = blockIdx.x; p < npatch; p += gridDim.x) {
-        const int64_t s0 = row_ptr[p];
-        const int nb = (int)(row_ptr[p + 1] - s0);
-        const int n = nb * b, n16 = (n + 15) & ~15, mt = n16 >> 4, ntile = mt * (mt + 1) / 2;
-        constexpr int ldp = kPatchLds;
-        __syncthreads(); // the previous patch's reads of sm
-        int32_t *tab = reinterpret_cast<int32_t *>(sm);
-        const bool table = nb <= kPatchTab;
-        if (table)
-            for (int t = tid; t < nb * nb; t += 1024)
-                tab[t] = (int32_t)find_block(row_ptr, col_ind, col_ind[s0 + t / nb], col_ind[s0 + t % nb]);
-        __syncthreads();
-        // entry (r, c) of A, read as (c, r): its column-major block is
-        // contiguous along c for one r
-        auto entry = [&](int r, int c) -> double {
-            const int pb = r / b, rr = r - pb * b, q = c / b, cc = c - q * b;
-            const int64_t sb = table ? tab[q * nb + pb]
-                                     : find_block(row_ptr, col_ind, col_ind[s0 + q], col_ind[s0 + pb]);
-            return sb < 0 ? 0.0 : vals[sb * (int64_t)b * b + rr * b + cc];
-        };
-        // c = max_r sum_c |A_rc| (Gershgorin)
-        double mx = 0.0;
-        for (int r = wave; r < n; r += 16) {
-            double sum = 0.0;
-            for (int c = lane; c < n; c += 64) sum += fabs(entry(r, c));
-            mx = fmax(mx, wave_sum(sum));
-        }
-        mx = combine(mx, true);
-        const double c0 = mx > 0.0 ? mx : 1.0, inv = 1.0 / c0;
-        // Y0 = diag(A/c, I); Z0 = I, so the first update needs no product:
-        // Z1 = T0 = (3 I - Y0) / 2
-        double rs = 0.0;
-        for (int t = wave; t < ntile; t += 16) {
-            const int tr = tile_row(t), tc = t - tr * (tr + 1) / 2;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = 16 * tr + 4 * v + g, c = 16 * tc + i;
-                const double id = r == c ? 1.0 : 0.0;
-                const double y = r < n && c < n ? entry(r, c) * inv : id;
-                const double d = id - y;
-                rs = __builtin_fma(tr == tc ? d : 2.0 * d, d, rs);
-                Y[t * 256 + 64 * v + lane] = y;
-                Z[t * 256 + 64 * v + lane] = 1.5 * id - 0.5 * y;
-            }
-        }
-        double res = sqrt(combine(wave_sum(rs), false));
-
-        // C = A B, or C = 1.5 I - 0.5 A B with the residual's sum of squares
-        // returned (T0); C may be A or B. N tiles a wave, the last one of some
-        // waves a repeat of the last tile: no branch between the MFMAs.
-        auto product = [&](auto n_c, const double *A, const double *B, double *C, bool t0) -> double {
-            constexpr int N = decltype(n_c)::value;
-            D4 acc[N];
-#pragma unroll
-            for (int q = 0; q < N; ++q) acc[q] = D4{0, 0, 0, 0};
-            // this wave's tiles wave, wave + 16, ...: this lane's places in the panels
-            int ta[N], tb[N];
-#pragma unroll
-            for (int q = 0; q < N; ++q) {
-                const int t = min(wave + 16 * q, ntile - 1), tr = tile_row(t);
-                ta[q] = g * ldp + i + 16 * tr;
-                tb[q] = (16 + g) * ldp + i + 16 * (t - tr * (tr + 1) / 2);
-            }
-            // Chunk tk of an operand, its rows 16 tk .. 16 tk + 15, is the tiles
-            // (tk, j <= tk) and, transposed, (j > tk, tk): 128 pieces of 16 bytes a
-            // tile, at most two a thread. Transposed tiles are read down their
-            // columns, so that their LDS writes are 16 consecutive values.
-            const int e = tid & 127;
-            const int j0 = __builtin_amdgcn_readfirstlane(tid >> 7), j1 = j0 + 8;
-            const bool p0 = j0 < mt, p1 = j1 < mt;
-            auto where = [&](int j, int tk) -> int {
-                return j <= tk ? (tk * (tk + 1) / 2 + j) * 256 + 2 * e
-                               : (j * (j + 1) / 2 + tk) * 256 + (e & 15) * 16 + 2 * (e >> 4);
-            };
-            double2 ra0, ra1, rb0, rb1;
-            auto fetch = [&](int tk) { // threads past the chunk read its last tile
-                const int o0 = where(p0 ? j0 : mt - 1, tk), o1 = where(p1 ? j1 : mt - 1, tk);
-                ra0 = *reinterpret_cast<const double2 *>(A + o0);
-                rb0 = *reinterpret_cast<const double2 *>(B + o0);
-                ra1 = *reinterpret_cast<const double2 *>(A + o1);
-                rb1 = *reinterpret_cast<const double2 *>(B + o1);
-            };
-            auto put = [&](double *d, int j, int tk, double2 v) {
-                if (j <= tk) {
-                    *reinterpret_cast<double2 *>(d + (e >> 3) * ldp + 16 * j + 2 * (e & 7)) = v;
-                } else {
-                    d += 2 * (e >> 4) * ldp + 16 * j + (e & 15);
-                    d[0] = v.x;
-                    d[ldp] = v.y;
-                }
-            };
-            auto stage = [&](int buf, int tk) {
-                double *d = sm + buf * 32 * kPatchLds, *dB = d + 16 * ldp;
-                if (p0) {
-                    put(d, j0, tk, ra0);
-                    put(dB, j0, tk, rb0);
-                }
-                if (p1) {
-                    put(d, j1, tk, ra1);
-                    put(dB, j1, tk, rb1);
-                }
-            };
-            __syncthreads(); // A and B are written, sm is free
-            fetch(0);
-            stage(0, 0);
-            __syncthreads();
-            for (int tk = 0; tk < mt; ++tk) {
-                const int buf = tk & 1;
-                const bool more = tk + 1 < mt;
-                const double *panel = sm + buf * 32 * ldp;
-                // the chunk's 4 N MFMAs in order, each one's operands read two
-                // MFMAs ahead (left to itself the compiler reads, waits and
-                // multiplies in turn); the next chunk's loads and LDS writes go
-                // in between, so that only a barrier and an LDS read lie
-                // between two chunks' MFMAs
-                double fa[3], fb[3];
-                auto frag = [&](int m) {
-                    fa[m % 3] = panel[m / N * 4 * ldp + ta[m % N]];
-                    fb[m % 3] = panel[m / N * 4 * ldp + tb[m % N]];
-                };
-                frag(0);
-                if (4 * N > 1) frag(1);
-#pragma unroll
-                for (int m = 0; m < 4 * N; ++m) {
-                    if (m + 2 < 4 * N) frag(m + 2);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (m == 1 && more) fetch(tk + 1);
-                    if (m == (N > 1 ? 3 * N : 2) && more) stage(buf ^ 1, tk + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    acc[m % N] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[m % 3], fb[m % 3], acc[m % N], 0, 0, 0);
-                }
-                __syncthreads();
-            }
-            // the tiles, 512 consecutive bytes a store; one on the diagonal
-            // takes its upper half from its lower one, through this wave's own
-            // 16 x 17 piece of LDS
-            double sq = 0.0;
-            double *tile = sm + wave * 16 * 17;
-#pragma unroll
-            for (int q = 0; q < N; ++q)
-                if (wave + 16 * q < ntile) {
-                    const bool diag = ta[q] + 16 * ldp == tb[q];
-                    if (diag) {
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) tile[(4 * v + g) * 17 + i] = acc[q][v];
-                        __builtin_amdgcn_wave_barrier();
-                    }
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int lr = 4 * v + g; // f64 accumulator layout
-                        double x = acc[q][v];
-                        if (diag && i > lr) x = tile[i * 17 + lr];
-                        if (t0) {
-                            const double id = diag && i == lr ? 1.0 : 0.0, d = id - x;
-                            sq = __builtin_fma(diag ? d : 2.0 * d, d, sq);
-                            x = 1.5 * id - 0.5 * x;
-                        }
-                        C[(wave + 16 * q) * 256 + 64 * v + lane] = x;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                }
-            return t0 ? sqrt(combine(wave_sum(sq), false)) : 0.0;
-        };
-
-        // the products of the iteration, one call for all: Y1 = Y0 T0, then
-        // T = (3 I - Z Y) / 2, Y = Y T, Z = T Z until T's residual ends it
-        int it = 0;
-        bool conv = res < tol;
-        if (!conv && res <= 100.0 && it < maxit)
-            for (int op = 0;; op = op == 0 || op == 3 ? 1 : op + 1) {
-                const double *A = op == 1 ? Z : op == 3 ? T : Y, *B = op == 1 ? Y : op == 2 ? T : Z;
-                double *C = op == 1 ? T : op == 3 ? Z : Y;
-                double r = 0.0;
-#define RG_NS_CASE(N_)                                                                                       \
-    case N_:                                                                                                 \
-        if constexpr (N_ <= NQ) r = product(std::integral_constant<int, N_>{}, A, B, C, op == 1);            \
-        break;
-                switch ((ntile + 15) >> 4) {
-                    RG_NS_CASE(1)
-                    RG_NS_CASE(2)
-                    RG_NS_CASE(3)
-                    RG_NS_CASE(4)
-                    RG_NS_CASE(5)
-                    RG_NS_CASE(6)
-                    RG_NS_CASE(7)
-                    RG_NS_CASE(8)
-                    RG_NS_CASE(9)
-                }
-#undef RG_NS_CASE
-                if (op != 1) continue;
-                ++it;
-                res = r;
-                conv = res < tol;
-                if (conv || !(res <= 100.0) || it == maxit) break;
-            }
-        if (tid == 0) {
-            iters[p] = it;
-            resid[p] = res;
-        }
-        if (!conv) continue; // the host reports it
-        __syncthreads();
-        // block row i: rows of block i of T Z / sqrt(c) (Z0 = I: of T0), T's rows in LDS
-        int me = 0;
-        for (int q = 0; q < nb; ++q)
-            if (col_ind[s0 + q] == (int32_t)p) me = q;
-        const double *Tm = it == 0 ? Z : T;
-        for (int t = tid; t < b * n16; t += 1024) sm[t] = at(Tm, me * b + t / n16, t % n16);
-        __syncthreads();
-        const double sc = 1.0 / sqrt(c0);
-        const int c = tid & 255, rg0 = tid >> 8; // rows rg0, rg0 + 4, ...
-        if (c < n) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-            if (it == 0) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (rg0 + 4 * k < b) acc[k] = sm[(rg0 + 4 * k) * n16 + c];
-            } else {
-                for (int k = 0; k < n; ++k) {
-                    const double z = at(Z, k, c);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (rg0 + 4 * q < b) acc[q] = __builtin_fma(sm[(rg0 + 4 * q) * n16 + k], z, acc[q]);
-                }
-            }
-            const int q = c / b, cc = c - q * b;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (rg0 + 4 * k < b) zout[(s0 + q) * (int64_t)b * b + cc * b + rg0 + 4 * k] = acc[k] * sc;
-        }
-    }
-}
-
 // Z block row i = rows of block i in Zp / sqrt(c), into column-major blocks.
 __global__ __launch_bounds__(256) void k_patch_extract(int64_t first, int b,
                                                        const int64_t *__restrict__ row_ptr,
@@ -606,6 +271,12 @@ __device__ __forceinline__ D4 mm16(const double *A, const double *B, int i, int 
 __device__ __forceinline__ void st16(double *D, D4 v, int i, int g) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) D[(4 * q + g) * SPL + i] = v[q];
+}
+
+__device__ __forceinline__ double wave_sum(double x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
 }
 
 __device__ __forceinline__ double wave_max(double x) {
@@ -846,44 +517,6 @@ hipError_t launch_patch_gather(int64_t first, int64_t count, int b, const int64_
     hipLaunchKernelGGL(k_patch_gather, dim3((unsigned)count), dim3(256), 0, st, first, b, row_ptr,
                        col_ind, vals, ld, Y, Z, cs);
     return hipGetLastError();
-}
-
-hipError_t launch_asymmetric(int64_t nbr, int b, const int64_t *row_ptr, const int32_t *col_ind, const double *vals,
-                             int *flag, hipStream_t st) {
-    hipLaunchKernelGGL(k_asymmetric, dim3((unsigned)(nbr < 16384 ? nbr : 16384)), dim3(256), 0, st, nbr, b, row_ptr,
-                       col_ind, vals, flag);
-    return hipGetLastError();
-}
-
-int ns_patch_max() { return kPatchMax; }
-
-// One workgroup per compute unit (its LDS holds one), fewer for few patches.
-int ns_patch_grid(int64_t npatch) {
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
-        ncu = 256;
-    return (int)(npatch < ncu ? npatch : ncu);
-}
-
-size_t ns_patch_bytes(int grid, int ld) {
-    const int mt = ld / 16;
-    return (size_t)grid * 3 * (mt * (mt + 1) / 2) * 256 * 8;
-}
-
-hipError_t launch_ns_patch(int64_t npatch, int grid, int b, const int64_t *row_ptr, const int32_t *col_ind,
-                           const double *vals, int ld, double tol, int maxit, double *work, double *zout, int *iters,
-                           double *resid, hipStream_t st) {
-    if (ld % 16 != 0 || ld < 16 || ld > kPatchMax || b < 1 || b > 16 || grid < 1) return hipErrorInvalidValue;
-    const int mt = ld / 16, ldt = mt * (mt + 1) / 2, nq = (ldt + 15) / 16;
-    auto go = [&](auto nq_c) {
-        hipLaunchKernelGGL((k_ns_patch<decltype(nq_c)::value>), dim3(grid), dim3(1024), 0, st, npatch, b, row_ptr,
-                           col_ind, vals, ldt, tol, maxit, work, zout, iters, resid);
-        return hipGetLastError();
-    };
-    if (nq <= 4) return go(std::integral_constant<int, 4>{});
-    if (nq <= 7) return go(std::integral_constant<int, 7>{});
-    return go(std::integral_constant<int, 9>{});
 }
 
 hipError_t launch_ns_gemm(int mode, int64_t count, int ld, const double *A, const double *B,
