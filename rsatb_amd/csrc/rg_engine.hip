@@ -447,11 +447,17 @@ std::vector<int32_t> d2_colouring(int64_t n, const int64_t *rp, const int32_t *c
             for (int64_t p = rp[r]; p < rp[r + 1]; ++p) tr[(size_t)pos[(size_t)ci[p]]++] = (int32_t)r;
     }
     std::vector<int32_t> col((size_t)n, -1);
-    // the colours taken in every row, nw words of 64 a row: a column's choice is
+    // The colours taken in every row, nw words of 64 a row: a column's choice is
     // the lowest bit clear in all its rows (walking the rows' columns instead took
-    // 17 times the reads at 17 blocks a row)
+    // 17 times the reads at 17 blocks a row). The words double up to kColourWords;
+    // a colour past them is found by the walk, so a dense row costs what its
+    // walks cost and no words in the other rows (one row of 40,000 columns: 1.5 s
+    // and 3 MB; with words for all its colours 42 s and 200 MB).
+    constexpr size_t kColourWords = 8;
     size_t nw = 1;
     std::vector<uint64_t> used((size_t)n, 0);
+    std::vector<int64_t> mark; // mark[k] == stamp: colour 64 kColourWords + k is taken near the column
+    int64_t stamp = 0;
     for (int32_t r : order)
         for (int64_t p = rp[r]; p < rp[r + 1]; ++p) {
             const int32_t c = ci[p];
@@ -464,13 +470,29 @@ std::vector<int32_t> d2_colouring(int64_t n, const int64_t *rp, const int32_t *c
                 for (int64_t t = t0; t < t1; ++t) m |= used[(size_t)tr[(size_t)t] * nw + w];
                 if (~m) break;
             }
+            if (w == kColourWords) {
+                ++stamp;
+                for (int64_t t = t0; t < t1; ++t) {
+                    const int32_t rr = tr[(size_t)t];
+                    for (int64_t q = rp[rr]; q < rp[rr + 1]; ++q) {
+                        const int64_t k = col[(size_t)ci[q]] - (int64_t)(64 * kColourWords);
+                        if (k < 0) continue;
+                        if ((size_t)k >= mark.size()) mark.resize((size_t)k + 1, 0);
+                        mark[(size_t)k] = stamp;
+                    }
+                }
+                size_t k = 0;
+                while (k < mark.size() && mark[k] == stamp) ++k;
+                col[(size_t)c] = (int32_t)(64 * kColourWords + k);
+                continue;
+            }
             if (w == nw) {
-                std::vector<uint64_t> wider((size_t)n * (nw + 1), 0);
+                std::vector<uint64_t> wider((size_t)n * 2 * nw, 0);
                 for (size_t i = 0; i < (size_t)n; ++i)
                     std::copy(used.begin() + (ptrdiff_t)(i * nw), used.begin() + (ptrdiff_t)((i + 1) * nw),
-                              wider.begin() + (ptrdiff_t)(i * (nw + 1)));
+                              wider.begin() + (ptrdiff_t)(i * 2 * nw));
                 used.swap(wider);
-                ++nw;
+                nw *= 2;
                 m = 0;
             }
             const int bit = __builtin_ctzll(~m);
