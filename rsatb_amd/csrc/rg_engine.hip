@@ -2318,7 +2318,7 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
         Kc = std::max<size_t>(1, std::min(K, budget / (2 * (size_t)M * 8 * cw)));
         RG_HIP(ctx, ctx->kg_work.ensure(2 * (size_t)M * Kc * 8 * cw), "hipMalloc widening panels");
     }
-    const KgGemmPlan gp = kg_gemm_plan(M, (int64_t)K);
+    const KgGemmPlan gp = kg_gemm_plan(M, (int64_t)K, np);
     if (!vm.complex_vec) RG_HIP(ctx, ctx->kg_part.ensure(kg_gemm_bytes(gp, np)), "hipMalloc moment parts");
     auto timed = [&](int products, auto run) -> int { // run() as one launch of the product class
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -2357,7 +2357,8 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
             }
             return timed(np, [&]() -> int {
                 RG_HIP(ctx, launch_kg_gemm(gp, p, np, fp32, (int64_t)K, (int64_t)Kp, M, s2, beta_in,
-                                           static_cast<double *>(ctx->kg_part.p), out, (int64_t)mm, ctx->stream),
+                                           static_cast<double *>(ctx->kg_part.p), ctx->kg_part.bytes, out, (int64_t)mm,
+                                          ctx->stream),
                        "moment products");
                 return RG_OK;
             });

@@ -288,7 +288,7 @@ hipError_t launch_kg_moment(const BsrDev &H, VecMode vm, const KgMoment &a, int 
 hipError_t launch_same_pattern(const BsrDev &A, const BsrDev &B, int *flag, hipStream_t st);
 // real moment products out[q] = alpha l[q]^T r[q] + beta out[q] (column-major
 // M x M each, out_stride apart) of sequences of M vectors of K elements, ld apart
-// (16-byte aligned); part holds kg_gemm_bytes
+// (16-byte aligned); part_bytes >= kg_gemm_bytes
 struct KgGemm {
     const void *l[6], *r[6];
 };
@@ -296,13 +296,14 @@ struct KgGemmPlan {
     int a = 4, nt = 1, nchunk = 1;
     int64_t kc = 16;
 };
-KgGemmPlan kg_gemm_plan(int M, int64_t K);
+KgGemmPlan kg_gemm_plan(int M, int64_t K, int npairs);
 inline size_t kg_gemm_bytes(const KgGemmPlan &p, int npairs) {
     const size_t side = (size_t)p.nt * 32 * p.a;
     return (size_t)npairs * p.nchunk * side * side * 8;
 }
 hipError_t launch_kg_gemm(const KgGemmPlan &pl, const KgGemm &p, int npairs, bool fp32, int64_t K, int64_t ld, int M,
-                          double alpha, double beta, double *part, double *out, int64_t out_stride, hipStream_t st);
+                          double alpha, double beta, double *part, size_t part_bytes, double *out, int64_t out_stride,
+                          hipStream_t st);
 // node weights GC, GE, GNE ([m + k M] complex each) from the damping g[m]
 hipError_t launch_kg_weights(int M, const double *g, double2 *W, hipStream_t st);
 hipError_t launch_kg_widen(const double *in, bool cplx, double2 *out, int64_t n, hipStream_t st);

@@ -136,15 +136,21 @@ __global__ __launch_bounds__(256) void k_kg_moment(int64_t n, int ulen, const in
 // K elements in 16-byte accesses, so a row's four lane groups load 64 contiguous
 // bytes each time (FP32 is widened in registers: products of two FP32 values
 // are exact), and four MFMAs take one element each; no LDS. Rows lie ld
-// apart and have at least sixteen elements of memory. The tiles of a chunk run on
-// one XCD, whose L2 holds the chunk's rows. Bound by the MFMAs (M^2 K / 36.6
-// TF/s) above M of about 100, by reading the sequences below.
+// apart and have at least sixteen elements of memory. An XCD takes a contiguous
+// eighth of a product's (chunk, tile) list, so that its L2 holds the rows of few
+// chunks, or of a strip of tiles, and no XCD idles when there are fewer chunks than
+// XCDs (a chunk to an XCD: M = 1,024 33 TF/s, M = 1,500 and above 8). Bound by the
+// MFMAs (M^2 K / 36.6 TF/s) above M of about 100, by reading the sequences below.
 // Measured, three products, against rocBLAS, which cuts K only for some sizes:
-// M = 256, K = 1,048,576 7.5 -> 7.0 ms; M = 200 7.0 -> 7.5; M = 90, K = 409,600
-// 2.35 -> 0.47; M = 128, K = 120,000 58 -> 0.22; M = 512, K = 131,072 63 -> 3.5;
-// M = 1024, K = 73,728 36 -> 14; M = 64, K = 4,096 0.67 -> 0.01. Vectors a power of
-// two apart took 10.6 instead of 9.6 ms, a masked tail of scalar loads in the
-// loop 9.6 instead of 7.0. Error of the moments against 80-bit sums (rel. 2-norm),
+// M = 64, K = 4,096 0.67 -> 0.014 ms; M = 90, K = 409,600 2.35 -> 0.52; M = 128, K =
+// 120,000 58 -> 0.25; M = 200, K = 262,144 1.72 -> 1.68; M = 256 1.80 -> 1.71; M = 512,
+// K = 131,072 63 -> 3.6; M = 1,024, K = 73,728 36 -> 8.0; M = 1,500, K = 65,536 32 ->
+// 16.1; M = 2,048, K = 32,768 16.7 -> 13.9; M = 4,096, K = 16,384 26.2 -> 26.6, K =
+// 2,048 3.3 -> 4.0 (one chunk's parts are written and read again; storing the
+// results from here instead moved the accumulators between the register files
+// and took 46 in place of 58 TF/s at every size). Vectors a power of two apart took
+// 10.6 instead of 9.6 ms (M = 256, K = 1,048,576), a masked tail of scalar loads in
+// the loop 9.6 instead of 7.0. Error of the moments against 80-bit sums (rel. 2-norm),
 // library / here: K = 36,000, M = 128 5.1e-15 / 2.9e-16; K = 96,000, M = 96
 // 8.7e-15 / 2.0e-16: shorter chains of additions.
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -155,17 +161,25 @@ __global__ __launch_bounds__(256, 1) void k_kg_gemm(KgGemm p, int64_t K, int64_t
     constexpr int T = 32 * A;
     constexpr int E = 16 / (int)sizeof(S), P = 4 / E; // elements of an access, accesses a row
     typedef S SE __attribute__((ext_vector_type(E), aligned(sizeof(S))));
-    const int tiles = nt * nt, rest = (int)blockIdx.x >> 3;
-    const int tile = rest % tiles, chunk = (rest / tiles) * 8 + ((int)blockIdx.x & 7);
-    if (chunk >= nchunk) return;
+    // a product's items in the order (chunk, tile); every XCD takes a contiguous
+    // eighth, another one in each product, as the eighths differ by an item
+    const int tiles = nt * nt, items = tiles * nchunk, pair = (int)blockIdx.y;
+    const int xcd = ((int)blockIdx.x + pair) & 7;
+    const int item = (int)((int64_t)items * xcd / 8) + ((int)blockIdx.x >> 3);
+    if (item >= (int)((int64_t)items * (xcd + 1) / 8)) return;
+    const int chunk = item / tiles, tile = item - chunk * tiles;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = lane & 15, g = lane >> 4;
-    const int m0 = (tile / nt) * T + (wave >> 1) * 16 * A, n0 = (tile % nt) * T + (wave & 1) * 16 * A;
-    const S *__restrict__ lp[A], *__restrict__ rp[A];
+    // rows of the product are right vectors n, columns left vectors m, so that
+    // the parts and mu (column-major) lie alike
+    // tiles go down strips of four rows: 32 in flight on an XCD read 12 panels
+    const int strip = tile / (4 * nt), high = min(4, nt - 4 * strip), along = tile - strip * 4 * nt;
+    const int n0 = (4 * strip + along % high) * T + (wave >> 1) * 16 * A, m0 = (along / high) * T + (wave & 1) * 16 * A;
+    const S *__restrict__ rp[A], *__restrict__ lp[A];
 #pragma unroll
-    for (int r = 0; r < A; ++r) { // rows past M load the last one and are not stored
-        lp[r] = static_cast<const S *>(p.l[blockIdx.y]) + (int64_t)min(m0 + 16 * r + i, M - 1) * ld;
-        rp[r] = static_cast<const S *>(p.r[blockIdx.y]) + (int64_t)min(n0 + 16 * r + i, M - 1) * ld;
+    for (int r = 0; r < A; ++r) { // vectors past M load the last one and are not stored
+        rp[r] = static_cast<const S *>(p.r[pair]) + (int64_t)min(n0 + 16 * r + i, M - 1) * ld;
+        lp[r] = static_cast<const S *>(p.l[pair]) + (int64_t)min(m0 + 16 * r + i, M - 1) * ld;
     }
     const int64_t k0 = chunk * kc, k1 = min(K, k0 + kc);
     d4 acc[A][A];
@@ -182,8 +196,8 @@ __global__ __launch_bounds__(256, 1) void k_kg_gemm(KgGemm p, int64_t K, int64_t
         for (int r = 0; r < A; ++r)
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const SE x = *reinterpret_cast<const SE *>(lp[r] + kk + 4 * E * q);
-                const SE y = *reinterpret_cast<const SE *>(rp[r] + kk + 4 * E * q);
+                const SE x = *reinterpret_cast<const SE *>(rp[r] + kk + 4 * E * q);
+                const SE y = *reinterpret_cast<const SE *>(lp[r] + kk + 4 * E * q);
 #pragma unroll
                 for (int j = 0; j < E; ++j) {
                     a[r][E * q + j] = (double)x[j];
@@ -222,16 +236,16 @@ __global__ __launch_bounds__(256, 1) void k_kg_gemm(KgGemm p, int64_t K, int64_t
         }
     }
     const int64_t Mp = (int64_t)nt * T;
-    double *__restrict__ out = part + ((int64_t)blockIdx.y * nchunk + chunk) * Mp * Mp;
+    double *__restrict__ out = part + ((int64_t)pair * nchunk + chunk) * Mp * Mp;
 #pragma unroll
     for (int r = 0; r < A; ++r)
 #pragma unroll
         for (int c = 0; c < A; ++c)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) out[(int64_t)(m0 + 16 * r + 4 * v + g) * Mp + n0 + 16 * c + i] = acc[r][c][v];
+            for (int v = 0; v < 4; ++v) out[(int64_t)(n0 + 16 * r + 4 * v + g) * Mp + m0 + 16 * c + i] = acc[r][c][v];
 }
 
-// out[m + n M] = alpha sum over the chunks of part[m][n] + beta out[m + n M]:
+// out[n M + m] = alpha sum over the chunks of part[n][m] + beta out[n M + m]:
 // 64 elements a workgroup, four threads each taking every fourth chunk.
 __global__ __launch_bounds__(256) void k_kg_sum(const double *__restrict__ part, int nchunk, int Mp, int M,
                                                 double alpha, double beta, double *__restrict__ out,
@@ -239,17 +253,17 @@ __global__ __launch_bounds__(256) void k_kg_sum(const double *__restrict__ part,
     __shared__ double sm[4][64];
     const int u = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int64_t e = (int64_t)blockIdx.x * 64 + u, mat = (int64_t)Mp * Mp;
-    const int m = (int)(e / M), n = (int)(e - (int64_t)m * M);
+    const int n = (int)(e / M), m = (int)(e - (int64_t)n * M);
     double s = 0.0;
-    if (m < M) {
-        const double *q = part + (int64_t)blockIdx.y * nchunk * mat + (int64_t)m * Mp + n;
+    if (n < M) {
+        const double *q = part + (int64_t)blockIdx.y * nchunk * mat + (int64_t)n * Mp + m;
 #pragma unroll 8
         for (int c = w; c < nchunk; c += 4) s += q[c * mat];
     }
     sm[w][u] = s;
     __syncthreads();
-    if (w == 0 && m < M) {
-        double *o = out + blockIdx.y * out_stride + (int64_t)n * M + m;
+    if (w == 0 && n < M) {
+        double *o = out + blockIdx.y * out_stride + e;
         const double v = alpha * (sm[0][u] + sm[1][u] + sm[2][u] + sm[3][u]);
         *o = beta == 0.0 ? v : v + beta * *o;
     }
@@ -351,9 +365,15 @@ hipError_t launch_same_pattern(const BsrDev &A, const BsrDev &B, int *flag, hipS
     return hipGetLastError();
 }
 
-// Tile side: the fewest padded outputs, wider on a tie; chunks of K: one
-// workgroup a CU, at least 64 elements each.
-KgGemmPlan kg_gemm_plan(int M, int64_t K) {
+// Tile side: the fewest padded outputs, wider on a tie. Chunks of K: at least 64
+// elements each, one workgroup a CU of every product while that gives eight or
+// more (two where the tiles are narrow). With fewer the last round of workgroups
+// counts: the fewest chunks within 5 % of the least time, in K elements, where a
+// workgroup takes kc + 24 (its first loads wait), the rounds of workgroups end a
+// quarter of one late (one round of 243 on 256 CUs took two), and a workgroup's
+// part of the output, written and summed, is a round of 96. Measured, three
+// products, K = 65,536: M = 1,100 one chunk 28 TF/s, three 51.
+KgGemmPlan kg_gemm_plan(int M, int64_t K, int npairs) {
     KgGemmPlan p;
     int64_t best = 0;
     for (int a = 4; a >= 2; --a) {
@@ -364,17 +384,33 @@ KgGemmPlan kg_gemm_plan(int M, int64_t K) {
         }
     }
     p.nt = (int)(best / (32 * p.a));
-    const int64_t tiles = (int64_t)p.nt * p.nt;
-    const int64_t want = std::max<int64_t>(1, std::min<int64_t>((p.a == 4 ? 256 : 512) / tiles, (K + 63) / 64));
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
+        ncu = 256;
+    const int64_t tiles = (int64_t)p.nt * p.nt, slots = p.a == 4 ? ncu : 2 * ncu, most = (K + 63) / 64;
+    int64_t want = std::max<int64_t>(1, std::min<int64_t>(slots / tiles, most));
+    if (slots / tiles < 8) {
+        auto time = [&](int64_t c) {
+            const int64_t wgs = c * tiles * npairs, rounds = (wgs + slots - 1) / slots;
+            return ((double)rounds + 0.25) * ((double)K / c + 24.0) + 96.0 * wgs / slots;
+        };
+        const int64_t top = std::min<int64_t>(8, most);
+        double least = time(1);
+        for (int64_t c = 2; c <= top; ++c) least = std::min(least, time(c));
+        for (want = 1; time(want) > 1.05 * least;) ++want;
+    }
     p.kc = ((K + want - 1) / want + 15) / 16 * 16;
     p.nchunk = (int)((K + p.kc - 1) / p.kc);
     return p;
 }
 
 hipError_t launch_kg_gemm(const KgGemmPlan &pl, const KgGemm &p, int npairs, bool fp32, int64_t K, int64_t ld, int M,
-                          double alpha, double beta, double *part, double *out, int64_t out_stride, hipStream_t st) {
+                          double alpha, double beta, double *part, size_t part_bytes, double *out, int64_t out_stride,
+                          hipStream_t st) {
+    if (M < 1 || K < 1 || npairs < 1 || npairs > 6 || part_bytes < kg_gemm_bytes(pl, npairs)) return hipErrorInvalidValue;
     const int Mp = pl.nt * 32 * pl.a;
-    const dim3 grid((unsigned)((pl.nchunk + 7) / 8 * 8 * pl.nt * pl.nt), (unsigned)npairs);
+    const dim3 grid((unsigned)((pl.nchunk * pl.nt * pl.nt + 7) / 8 * 8), (unsigned)npairs);
 #define RG_KG_CASE(S_, A_)                                                                                          \
     hipLaunchKernelGGL((k_kg_gemm<S_, A_>), grid, dim3(256), 0, st, p, K, ld, pl.kc, M, pl.nt, pl.nchunk, part)
     if (fp32) {
