@@ -109,8 +109,10 @@ struct Slot {
     bool is_complex = false;
     DevBuf row_ptr, col_ind, vals64, vals32;
     bool vals32_valid = false;
-    // gather table of the MFMA SpMM: xrow[s * b + kk] = col_ind[s] * b + kk
+    // gather table of the MFMA SpMM (see BsrDev): the offsets (xoff_bytes), then
+    // the entries
     DevBuf xrow;
+    int64_t xlen = 0;
     bool has_xrow = false;
     // The MFMA SpMM's own view of the slot (real, b >= 8): block rows in a
     // processing order of compact regions of sreg rows (sched), and every
@@ -298,6 +300,9 @@ bool vec_complex(const rg_context *ctx) {
 
 size_t vec_elem_bytes(VecMode vm) { return (vm.complex_vec ? 2 : 1) * (vm.fp32 ? 4 : 8); }
 
+// Bytes of a gather table's offsets, in whole 16-byte pieces.
+size_t xoff_bytes(int64_t nbr) { return ((size_t)nbr + 2) / 2 * 16; }
+
 // True when the slot's MFMA view (the scheduled rows and colour-ordered
 // blocks) holds current values for the precision.
 bool plan_current(const Slot &s, bool fp32) {
@@ -316,16 +321,21 @@ BsrDev dev_view(const Slot &s, bool fp32) {
     d.is_complex = s.is_complex;
     d.ulen = s.ulen;
     d.maxlen = s.maxlen;
+    auto table = [&](const DevBuf &t) {
+        d.xoff = static_cast<const int64_t *>(t.p);
+        d.xrow = reinterpret_cast<const int32_t *>(static_cast<const char *>(t.p) + xoff_bytes(s.nbr));
+        d.xlen = s.xlen;
+    };
     if (plan_current(s, fp32)) {
         d.col_ind = static_cast<const int32_t *>(s.kcol.p);
         d.vals = fp32 ? s.kvals32.p : s.kvals64.p;
-        d.xrow = static_cast<const int32_t *>(s.kxrow.p);
+        table(s.kxrow);
         d.sched = static_cast<const int32_t *>(s.sched.p);
         return d;
     }
     d.col_ind = static_cast<const int32_t *>(s.col_ind.p);
     d.vals = fp32 ? s.vals32.p : s.vals64.p;
-    if (s.has_xrow) d.xrow = static_cast<const int32_t *>(s.xrow.p);
+    if (s.has_xrow) table(s.xrow);
     return d;
 }
 
@@ -539,11 +549,27 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
         if (r == s.nbr) s.ulen = (int32_t)rp[1];
     }
     if (s.b < 8) return RG_OK;
-    const int64_t n = s.nnzb * s.b;
     if ((int64_t)s.nbr * s.b > INT32_MAX) return RG_OK;
-    std::vector<int32_t> t((size_t)n + kXrowSpare, 0);
-    for (int64_t q = 0; q < s.nnzb; ++q)
-        for (int kk = 0; kk < s.b; ++kk) t[(size_t)(q * s.b + kk)] = ci[q] * s.b + kk;
+    // A ragged last step repeats the row's last X row: its A elements are zero,
+    // and another row's X could hold an infinity, which zero does not cancel.
+    auto steps4 = [&](int64_t r) { return ((rp[r + 1] - rp[r]) * s.b + 3) / 4 * 4; };
+    s.xlen = 0;
+    for (int64_t r = 0; r < s.nbr; ++r) s.xlen += steps4(r);
+    const size_t head = xoff_bytes(s.nbr) / 4; // of the offsets, in entries
+    std::vector<int32_t> t(head + (size_t)s.xlen + kXrowSpare, 0);
+    auto fill = [&](const int32_t *cols, const int32_t *order) {
+        int32_t *o = t.data() + head;
+        int64_t at = 0;
+        for (int64_t p = 0; p < s.nbr; ++p) {
+            std::memcpy(t.data() + 2 * p, &at, 8);
+            const int64_t r = order ? order[p] : p;
+            at += steps4(r);
+            for (int64_t q = rp[r]; q < rp[r + 1]; ++q)
+                for (int kk = 0; kk < s.b; ++kk) *o++ = cols[q] * s.b + kk;
+            for (; o < t.data() + head + at; ++o) *o = o[-1];
+        }
+    };
+    fill(ci, nullptr);
     RG_HIP(ctx, s.xrow.ensure(t.size() * 4), "hipMalloc gather table");
     RG_HIP(ctx, hipMemcpy(s.xrow.p, t.data(), t.size() * 4, hipMemcpyHostToDevice), "upload gather table");
     s.has_xrow = true;
@@ -551,10 +577,8 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     const int32_t sreg = ctx->mfma_sreg > 0 ? (int32_t)std::min<int64_t>(ctx->mfma_sreg, s.nbr) : plan_region_rows(s.nbr);
     MfmaPlan pl = mfma_plan(s.nbr, rp, ci, sreg);
     std::vector<int32_t> kc((size_t)s.nnzb + 1, 0);
-    for (int64_t q = 0; q < s.nnzb; ++q) {
-        kc[(size_t)q] = ci[pl.kperm[(size_t)q]];
-        for (int kk = 0; kk < s.b; ++kk) t[(size_t)(q * s.b + kk)] = kc[(size_t)q] * s.b + kk;
-    }
+    for (int64_t q = 0; q < s.nnzb; ++q) kc[(size_t)q] = ci[pl.kperm[(size_t)q]];
+    fill(kc.data(), pl.sched.data());
     RG_HIP(ctx, s.sched.ensure((size_t)s.nbr * 4), "hipMalloc row schedule");
     RG_HIP(ctx, s.kperm.ensure((size_t)s.nnzb * 4 + 4), "hipMalloc block order");
     RG_HIP(ctx, s.kcol.ensure(kc.size() * 4), "hipMalloc block order");
@@ -583,7 +607,8 @@ int copy_tables(rg_context *ctx, Slot &d, const Slot &src) {
     d.ulen = src.ulen;
     d.has_xrow = d.has_plan = false;
     d.kvals64_gen = d.kvals32_gen = 0;
-    const size_t nt = ((size_t)(src.nnzb * src.b) + kXrowSpare) * 4;
+    d.xlen = src.xlen;
+    const size_t nt = xoff_bytes(src.nbr) + ((size_t)src.xlen + kXrowSpare) * 4;
     if (src.has_xrow) RG_HIP(ctx, copy(d.xrow, src.xrow, nt), "copy gather table");
     if (src.has_plan) {
         RG_HIP(ctx, copy(d.sched, src.sched, (size_t)src.nbr * 4), "copy plan");
@@ -1193,7 +1218,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
         for (void *w : wv) key.push_back(addr(w));
         for (int sl = 0; sl < (ctx->form == RG_FORM_SANDWICH ? 3 : 1); ++sl) {
             const BsrDev q = dev_view(ctx->slots[sl], vm.fp32);
-            for (uint64_t x : {addr(q.row_ptr), addr(q.col_ind), addr(q.vals), addr(q.xrow), addr(q.sched),
+            for (uint64_t x : {addr(q.row_ptr), addr(q.col_ind), addr(q.vals), addr(q.xrow), addr(q.xoff), addr(q.sched),
                                (uint64_t)q.ulen, (uint64_t)q.nbr, (uint64_t)q.b, (uint64_t)q.nnzb,
                                (uint64_t)q.is_complex})
                 key.push_back(x);

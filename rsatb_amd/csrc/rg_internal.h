@@ -8,7 +8,7 @@ namespace rg {
 
 // Spare (zero) entries after the MFMA SpMM's gather table: a wave fetches up
 // to 2 PD - 2 steps of 4 entries past its row, and reads the entries of the
-// step after its last fetch (PD <= 8: at most 8 PD - 2 = 62 entries).
+// step after its last fetch (PD <= 8: 8 PD - 4 = 60 entries).
 constexpr int kXrowSpare = 64;
 
 // Device view of one BSR operand. Values are real (vals) or complex
@@ -21,9 +21,13 @@ struct BsrDev {
     const int32_t *col_ind = nullptr;
     const void *vals = nullptr; // double / double2 / float / float2
     bool is_complex = false;
-    // gather table of b >= 8 matrices, or null: xrow[s * b + kk] =
-    // col_ind[s] * b + kk, the X row of column kk of block s (kXrowSpare spare entries)
+    // gather table of b >= 8 matrices, or null: from xoff[p] on the X rows
+    // (col_ind[s] * b + kk of block s, column kk) of the columns of the block row
+    // at position p, in whole steps of four (a ragged last step repeats the row's
+    // last X row); xlen entries in all, then kXrowSpare spare ones
     const int32_t *xrow = nullptr;
+    const int64_t *xoff = nullptr;
+    int64_t xlen = 0;
     // processing order of the block rows (MFMA SpMM), or null for stored
     // order: position p of [0, nbr) computes block row sched[p]
     const int32_t *sched = nullptr;

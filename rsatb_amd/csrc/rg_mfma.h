@@ -385,6 +385,7 @@ template <typename S, int NT, int MODE, bool CV, bool CM> constexpr int prefetch
 template <typename S, int NT, int E, bool MASK, int MODE, bool CV, bool CM>
 __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spmm_mfma(int64_t nbr, int b,
                                                    const int64_t *__restrict__ row_ptr,
+                                                   const int64_t *__restrict__ xoff,
                                                    const int32_t *__restrict__ xrow,
                                                    const S *__restrict__ vals,
                                                    const S *__restrict__ zero,
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
     typedef S A2 __attribute__((ext_vector_type(2)));
     using AT = std::conditional_t<CM, A2, S>;
     constexpr int PD = prefetch_depth<S, NT, MODE, CV, CM>();
-    static_assert(8 * PD - 2 <= kXrowSpare, "the gather table's spare entries cover the fetches past a row");
+    static_assert(8 * PD - 4 <= kXrowSpare, "the gather table's spare entries cover the fetches past a row");
     static_assert(!CV || E % 2 == 0, "a complex column's halves share a lane");
     static_assert(!CM || CV, "complex matrices act on complex vectors");
     constexpr int NDOT = epi_ndot(MODE);
@@ -462,14 +463,14 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
         // scalar loads, so no vector load sits between the steps' loads). PD
         // register buffers: steps st + 1 .. st + PD - 1 are in flight while
         // step st's MFMAs run. Past the row's K the table still names a valid row
-        // and the panel read stays inside the padded value array; a = 0 there.
+        // (the row's own to the end of its last step); a = 0 there.
         // Lanes outside the panel (i >= b, or k >= K) load their A element from
         // `zero` (one element, 0) instead of selecting on loaded data, which
         // would hold up the next loads.
         const int K = nblk * b;
         const AT *__restrict__ panel = reinterpret_cast<const AT *>(vals) + s0 * (int64_t)b * b;
         int fst = 0; // next step to fetch
-        int64_t kb = s0 * b;
+        int64_t kb = xoff[pos];
         int32_t nx0 = xrow[kb], nx1 = xrow[kb + 1], nx2 = xrow[kb + 2], nx3 = xrow[kb + 3];
         auto fetch = [&](AT &a, S (&bv)[NT]) {
             // masks, not a select: the compiler branched over the lane groups
@@ -478,7 +479,7 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
             a = __builtin_nontemporal_load((i < b && k < K) ? panel + (int64_t)k * b + i
                                                             : reinterpret_cast<const AT *>(zero));
             load_cols<S, NT, E, MASK>(X + xr * W + col0, cm, bv);
-            // the next step's table entries (in range: the table keeps 8 PD - 2 <= 64 spare entries)
+            // the next step's table entries (in range: the table keeps 8 PD - 4 <= 64 spare entries)
             kb += 4;
             nx0 = xrow[kb];
             nx1 = xrow[kb + 1];
@@ -564,10 +565,10 @@ hipError_t go_mfma(const MfmaShape &s, const BsrDev &A, const void *X, void *Y, 
     // the zero element of lanes outside a panel: row_ptr[0] (0, checked when
     // a slot is written) for real values; for complex ones 16 aligned zero
     // bytes of the gather table's spare entries
-    const void *zero = CM ? static_cast<const void *>(A.xrow + (A.nnzb * A.b + 3) / 4 * 4)
+    const void *zero = CM ? static_cast<const void *>(A.xrow + A.xlen)
                           : static_cast<const void *>(A.row_ptr);
     hipLaunchKernelGGL((k_spmm_mfma<S, NT, E, MASK, MODE, CV, CM>), dim3(grid), dim3(64 * kMfmaWaves), 0, st, A.nbr,
-                       (int)A.b, A.row_ptr, A.xrow, static_cast<const S *>(A.vals), static_cast<const S *>(zero),
+                       (int)A.b, A.row_ptr, A.xoff, A.xrow, static_cast<const S *>(A.vals), static_cast<const S *>(zero),
                        static_cast<const S *>(X), static_cast<S *>(Y), W, R, s.nchunks, g_mfma.xcd_map, A.sched,
                        e);
     return hipGetLastError();
