@@ -91,7 +91,12 @@ struct DevBuf {
         }
         if (n == 0) n = 16;
         hipError_t e = hipMalloc(&p, n);
-        if (e == hipSuccess) bytes = n;
+        if (e == hipSuccess) {
+            bytes = n;
+        } else {
+            p = nullptr;
+            (void)hipGetLastError(); // not the next launch's error
+        }
         return e;
     }
     void release() {
@@ -257,11 +262,27 @@ int hipfail(rg_context *ctx, hipError_t e, const char *what) {
                 std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Frees what the context keeps only to save allocations; true when there was
+// something.
+bool give_back(rg_context *ctx) {
+    if (!ctx || !ctx->upload_staging.p) return false;
+    ctx->upload_staging.release();
+    return true;
+}
+
+// An allocation that finds no room is tried again after give_back (call is
+// then a DevBuf::ensure, which leaves nothing behind when it fails).
 #define RG_HIP(ctx, call, what)                                                                    \
     do {                                                                                           \
         hipError_t e_ = (call);                                                                    \
+        if (e_ == hipErrorOutOfMemory && give_back(ctx)) e_ = (call);                              \
         if (e_ != hipSuccess) return hipfail((ctx), e_, (what));                                   \
     } while (0)
+
+hipError_t ensure(rg_context *ctx, DevBuf &buf, size_t n) {
+    const hipError_t e = buf.ensure(n);
+    return e == hipErrorOutOfMemory && give_back(ctx) ? buf.ensure(n) : e;
+}
 
 hipEvent_t take_event(rg_context *ctx) {
     if (!ctx->pool.empty()) {
@@ -598,7 +619,7 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
 // are copies), copied on the device.
 int copy_tables(rg_context *ctx, Slot &d, const Slot &src) {
     auto copy = [&](DevBuf &to, const DevBuf &from, size_t bytes) {
-        hipError_t he = to.ensure(bytes);
+        hipError_t he = ensure(ctx, to, bytes);
         if (he == hipSuccess && bytes)
             he = hipMemcpyAsync(to.p, from.p, bytes, hipMemcpyDeviceToDevice, ctx->stream);
         return he;
@@ -1851,7 +1872,7 @@ int sk_build(rg_context *ctx, int slot, const rg_sk_table *t, int64_t n_atoms, c
     DevBuf &dints = ctx->sk_ints, &ddbl = ctx->sk_dbls, &dtype = ctx->sk_type, &dpos = ctx->sk_pos;
     DevBuf &dei = ctx->sk_ei, &dsh = ctx->sk_sh, &deblk = ctx->sk_eblk, &dflags = ctx->sk_flags;
     auto up = [&](DevBuf &d, const void *h, size_t bytes) -> hipError_t {
-        hipError_t e = d.ensure(bytes ? bytes : 16);
+        hipError_t e = ensure(ctx, d, bytes ? bytes : 16);
         if (e == hipSuccess && bytes) e = hipMemcpy(d.p, h, bytes, hipMemcpyHostToDevice);
         return e;
     };
@@ -1861,8 +1882,8 @@ int sk_build(rg_context *ctx, int slot, const rg_sk_table *t, int64_t n_atoms, c
     if (he == hipSuccess) he = up(dpos, pos, (size_t)n_atoms * 24);
     if (he == hipSuccess) he = up(dei, edge_index, (size_t)n_edges * 8);
     if (he == hipSuccess) he = up(dsh, edge_shift, (size_t)n_edges * 12);
-    if (he == hipSuccess) he = deblk.ensure((size_t)std::max<int64_t>(n_edges, 1) * b * b * 8);
-    if (he == hipSuccess) he = dflags.ensure((size_t)std::max<int64_t>(n_edges, 1));
+    if (he == hipSuccess) he = ensure(ctx, deblk, (size_t)std::max<int64_t>(n_edges, 1) * b * b * 8);
+    if (he == hipSuccess) he = ensure(ctx, dflags, (size_t)std::max<int64_t>(n_edges, 1));
     if (he != hipSuccess) return hipfail(ctx, he, "sk assemble: upload");
     SkDev sd;
     sd.n_types = T;
@@ -1990,9 +2011,9 @@ int sk_build(rg_context *ctx, int slot, const rg_sk_table *t, int64_t n_atoms, c
         s.vals32_valid = false;
         touch_slot(ctx, s);
         he = up(dph, w.data(), w.size() * 8);
-        if (he == hipSuccess) he = s.row_ptr.ensure((size_t)(n_atoms + 1) * 8);
-        if (he == hipSuccess) he = s.col_ind.ensure((size_t)nnzb * 4 + 4);
-        if (he == hipSuccess) he = s.vals64.ensure(nv * 8);
+        if (he == hipSuccess) he = ensure(ctx, s.row_ptr, (size_t)(n_atoms + 1) * 8);
+        if (he == hipSuccess) he = ensure(ctx, s.col_ind, (size_t)nnzb * 4 + 4);
+        if (he == hipSuccess) he = ensure(ctx, s.vals64, nv * 8);
         if (he == hipSuccess)
             he = hipMemcpy(s.row_ptr.p, row_ptr.data(), (size_t)(n_atoms + 1) * 8, hipMemcpyHostToDevice);
         if (he == hipSuccess)

@@ -1,0 +1,41 @@
+"""Device memory that a context holds beside what a call needs: given back, bounded,
+or done without when there is no room."""
+import numpy as np
+import pytest
+
+from rsatb_amd import _lib
+from rsatb_amd.bsr import BSR
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+def ring_blocks(n, b, width, seed):
+    """Symmetric block rows of the diagonal and `width` neighbours a side."""
+    rng = np.random.default_rng(seed)
+    k = np.arange(n)
+    d = rng.standard_normal((n, b, b))
+    rows, cols, vals = [k], [k], [d + np.swapaxes(d, 1, 2)]
+    for s in range(1, width + 1):
+        v = rng.standard_normal((n, b, b))
+        rows += [k, (k + s) % n]
+        cols += [(k + s) % n, k]
+        vals += [v, np.swapaxes(v, 1, 2)]
+    return BSR.from_blocks(n, b, np.concatenate(rows), np.concatenate(cols), np.concatenate(vals))
+
+
+def test_upload_staging_is_given_back_when_memory_runs_out():
+    H = ring_blocks(6000, 13, 6, 1)  # 105 MB of values
+    x = np.random.default_rng(2).standard_normal((H.n_rows, 2))
+    with _lib.Context(0) as ctx:
+        ctx.upload_bsr(_lib.SLOT_H, H)
+        y = ctx.bsr_mult(_lib.SLOT_H, x)
+        held = ctx.mem_info()[0]
+        with pytest.raises(_lib.RsatbGpuError):
+            ctx.set_samples(1 << 31, 256, _lib.SAMPLES_RADEMACHER, 1)  # 4 TB: no card has it
+        assert ctx.mem_info()[0] - held > 100 * MB
+        # and the context goes on
+        assert np.array_equal(ctx.bsr_mult(_lib.SLOT_H, x), y)
+        ctx.upload_bsr(_lib.SLOT_S, H)
+        assert np.array_equal(ctx.bsr_mult(_lib.SLOT_S, x), y)
