@@ -177,6 +177,10 @@ struct rg_context {
     DevBuf dpart; // per-step dot partials of a run whose reductions are deferred
     // projected moments: rows sorted by group, chunk and group ranges, dots
     DevBuf pd_rows, pd_chunk, pd_grp, pd_partial, pd_out;
+    // dpart and pd_partial hold a run's dots: not to be given back
+    bool stores_busy = false;
+    // bytes a store may take that a call can do without (RG_STORE_MAX)
+    size_t store_max = (size_t)1 << 30;
     // Slater-Koster assembly scratch (kept between calls): table, atoms,
     // edges, edge blocks, flags, gather plan
     DevBuf sk_ints, sk_dbls, sk_type, sk_pos, sk_ei, sk_sh, sk_eblk, sk_flags, sk_sp, sk_src, sk_ph, sk_row;
@@ -262,12 +266,18 @@ int hipfail(rg_context *ctx, hipError_t e, const char *what) {
                 std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// Frees what the context keeps only to save allocations; true when there was
-// something.
+// Frees what the context keeps only to save allocations or launches; true when
+// there was something.
 bool give_back(rg_context *ctx) {
-    if (!ctx || !ctx->upload_staging.p) return false;
+    if (!ctx) return false;
+    bool any = ctx->upload_staging.p != nullptr;
     ctx->upload_staging.release();
-    return true;
+    if (!ctx->stores_busy) {
+        any = any || ctx->dpart.p || ctx->pd_partial.p;
+        ctx->dpart.release();
+        ctx->pd_partial.release();
+    }
+    return any;
 }
 
 // An allocation that finds no room is tried again after give_back (call is
@@ -283,6 +293,20 @@ hipError_t ensure(rg_context *ctx, DevBuf &buf, size_t n) {
     const hipError_t e = buf.ensure(n);
     return e == hipErrorOutOfMemory && give_back(ctx) ? buf.ensure(n) : e;
 }
+
+// True when buf holds n bytes; false when that is more than a store may take or
+// than there is, and the call does without.
+bool store(rg_context *ctx, DevBuf &buf, size_t n) {
+    return n <= ctx->store_max && ensure(ctx, buf, n) == hipSuccess;
+}
+
+// While it lives the stores are in use.
+struct StoresScope {
+    rg_context *c;
+    bool was;
+    StoresScope(rg_context *ctx, bool in_use) : c(ctx), was(ctx->stores_busy) { c->stores_busy = was || in_use; }
+    ~StoresScope() { c->stores_busy = was; }
+};
 
 hipEvent_t take_event(rg_context *ctx) {
     if (!ctx->pool.empty()) {
@@ -1141,8 +1165,8 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     // and a b = 1 step over a million rows (90 us) still pays about 8 us for
     // it. Each doubled step then writes its dot partials to a region of its
     // own, and one batched launch after the loop reduces them all, in the
-    // same fixed order (the moments are the same bit for bit), whenever the
-    // regions of the whole run fit 1 GiB.
+    // same fixed order (the moments are the same bit for bit), whenever there is
+    // room for the regions of the whole run (at most store_max).
     const int chain_slot = ctx->form == RG_FORM_SANDWICH ? RG_SLOT_ZH : RG_SLOT_H;
     const int g_step = spmm_launch_grid(dev_view(ctx->slots[chain_slot], vm.fp32), vm, R);
     const int64_t pstride = (int64_t)g_step * 2 * R; // double2 per step region
@@ -1154,12 +1178,9 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     const bool onchip = ctx->onchip && doubled && !keep && !ctx->prof && ctx->form == RG_FORM_ORTHOGONAL &&
                         onchip_fits(dev_view(ctx->slots[RG_SLOT_H], vm.fp32), vm);
     const bool defer = doubled && !onchip && !noalloc && nsteps > 2 &&
-                       (size_t)nsteps * (size_t)pstride * 16 <= ((size_t)1 << 30);
-    double2 *dparts = nullptr;
-    if (defer) {
-        RG_HIP(ctx, ctx->dpart.ensure((size_t)nsteps * (size_t)pstride * 16), "hipMalloc step partials");
-        dparts = static_cast<double2 *>(ctx->dpart.p);
-    }
+                       store(ctx, ctx->dpart, (size_t)nsteps * (size_t)pstride * 16);
+    double2 *dparts = defer ? static_cast<double2 *>(ctx->dpart.p) : nullptr;
+    const StoresScope stores(ctx, defer);
 
     // forward states kept for the adjoint: psi_j for j <= 1 and j = 0, K-1 (mod K)
     ctx->ckpt_valid = false;
@@ -1401,6 +1422,7 @@ int rg_create(int device_id, rg_context **out) {
     if (const char *v = std::getenv("RG_GRAD_WIDE")) set_grad_wide(std::atoi(v));
     if (const char *v = std::getenv("RG_MFMA_PLAN")) ctx->mfma_plan = std::atoi(v) != 0;
     if (const char *v = std::getenv("RG_MFMA_SREG")) ctx->mfma_sreg = std::max(0, std::atoi(v));
+    if (const char *v = std::getenv("RG_STORE_MAX")) ctx->store_max = (size_t)std::max(0ll, std::atoll(v));
     if (const char *v = std::getenv("RG_KG_WIDEN_BYTES")) {
         const long long n = std::atoll(v);
         if (n > 0) ctx->kg_widen_bytes = (size_t)n;
@@ -1671,13 +1693,13 @@ int rg_kpm_pdos_moments(rg_context *ctx, int M, int precision, int doubling, int
     RG_HIP(ctx, ctx->pd_rows.ensure(rows.size() * 4), "hipMalloc group rows");
     RG_HIP(ctx, ctx->pd_chunk.ensure(chunk_ptr.size() * 8), "hipMalloc group chunks");
     RG_HIP(ctx, ctx->pd_grp.ensure(grp_chunk.size() * 8), "hipMalloc group chunks");
-    // a doubled run keeps every step's chunk dots and finishes them in one
-    // launch (the same sums in the same order) when they fit 1 GiB
-    const size_t part_bytes = (size_t)std::max<int64_t>(nchunks, 1) * 3 * 16;
-    const bool defer = doubled && part_bytes * (size_t)nsteps <= ((size_t)1 << 30);
-    RG_HIP(ctx, ctx->pd_partial.ensure(part_bytes * (defer ? (size_t)nsteps : 1)), "hipMalloc group partials");
     RG_HIP(ctx, ctx->pd_out.ensure((size_t)nsteps * 3 * std::max<int64_t>(G, 1) * 16),
            "hipMalloc group dots");
+    // a doubled run keeps every step's chunk dots and finishes them in one
+    // launch (the same sums in the same order) when there is room for them
+    const size_t part_bytes = (size_t)std::max<int64_t>(nchunks, 1) * 3 * 16;
+    const bool defer = doubled && store(ctx, ctx->pd_partial, part_bytes * (size_t)nsteps);
+    if (!defer) RG_HIP(ctx, ctx->pd_partial.ensure(part_bytes), "hipMalloc group partials");
     RG_HIP(ctx, hipMemcpy(ctx->pd_rows.p, rows.data(), rows.size() * 4, hipMemcpyHostToDevice),
            "upload group rows");
     RG_HIP(ctx, hipMemcpy(ctx->pd_chunk.p, chunk_ptr.data(), chunk_ptr.size() * 8,
@@ -1702,7 +1724,15 @@ int rg_kpm_pdos_moments(rg_context *ctx, int M, int precision, int doubling, int
     gd.bytes = 2.0 * (double)ngrouped * R * (double)vec_elem_bytes(vm);
 
     int nraw = 0;
+    const StoresScope stores(ctx, true);
     int rc = kpm_run(ctx, M, precision, doubling, total_out, nullptr, &gd, &nraw);
+    if (rc == RG_ERR_NOMEM && defer) { // the loop's own buffers need the room: step by step
+        ctx->pd_partial.release();
+        RG_HIP(ctx, ctx->pd_partial.ensure(part_bytes), "hipMalloc group partials");
+        gd.partial = static_cast<double2 *>(ctx->pd_partial.p);
+        gd.defer = false;
+        rc = kpm_run(ctx, M, precision, doubling, total_out, nullptr, &gd, &nraw);
+    }
     if (rc) return rc;
     if (G == 0) return RG_OK;
     std::vector<double2> host((size_t)nraw * 3 * G);

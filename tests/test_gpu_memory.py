@@ -39,3 +39,28 @@ def test_upload_staging_is_given_back_when_memory_runs_out():
         assert np.array_equal(ctx.bsr_mult(_lib.SLOT_H, x), y)
         ctx.upload_bsr(_lib.SLOT_S, H)
         assert np.array_equal(ctx.bsr_mult(_lib.SLOT_S, x), y)
+
+
+def test_projected_run_without_room_for_its_stores(monkeypatch):
+    """With no room for the chunk dots and dot partials of all steps a projected
+    run finishes step by step: the same sums in the same order."""
+    H = ring_blocks(4096, 9, 3, 3)
+    a = 1.1 * 9 * 7 * 3.0  # above the row sums' scale: any window does
+    groups = np.arange(H.n_rows) // 9
+    out, held = {}, {}
+    for limit in (None, str(MB)):
+        if limit:
+            monkeypatch.setenv("RG_STORE_MAX", limit)
+        with _lib.Context(0) as ctx:
+            ctx.upload_bsr(_lib.SLOT_H, H)
+            ctx.set_operator(_lib.FORM_ORTHOGONAL, 0.0, a)
+            ctx.set_samples(H.n_rows, 16, _lib.SAMPLES_RADEMACHER, 5)
+            free = ctx.mem_info()[0]
+            out[limit] = ctx.kpm_pdos_moments(512, groups, 4096)
+            held[limit] = free - ctx.mem_info()[0]
+            plain = ctx.kpm_moments(512)
+        assert np.array_equal(plain, out[limit][0])
+    for x, y in zip(out[None], out[str(MB)]):
+        assert np.array_equal(x, y)
+    # 4,096 chunks of 48 bytes in each of 257 steps
+    assert held[None] - held[str(MB)] > 40 * MB
