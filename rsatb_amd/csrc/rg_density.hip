@@ -52,10 +52,9 @@ __global__ __launch_bounds__(64) void k_density(const double *__restrict__ w, in
 
 int density_batch(int64_t G) { return G >= 8 ? 8 : 1; }
 
-hipError_t launch_density(const double *w, int64_t G, int M, const double *x, int64_t nx, double edge_inset,
+hipError_t launch_density(const double *w, int64_t G, int gb, int M, const double *x, int64_t nx, double edge_inset,
                           double *rho, hipStream_t st) {
-    if (G < 1 || M < 1 || nx < 1) return hipErrorInvalidValue;
-    const int gb = density_batch(G);
+    if (G < 1 || M < 1 || nx < 1 || (gb != 1 && gb != 8)) return hipErrorInvalidValue;
     const int64_t ny = (G + gb - 1) / gb, bx = (nx + 63) / 64;
     if (ny > 65535 || bx > INT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((unsigned)bx, (unsigned)ny);

@@ -3310,37 +3310,54 @@ int rg_kpm_density_batch(rg_context *ctx, const double *mu, int64_t G, int M, co
     std::vector<double> gk;
     if (kpm_weights(kernel, M, gk) != RG_OK) return fail(ctx, RG_ERR_INVALID, "unknown kernel");
     const int gb = density_batch(G);
-    // Few terms stay on the host: a launch with its transfers costs about
-    // 45 us, the host loop 2.2 ns a term.
-    if ((double)G * M * nx < 2e4 || (G + gb - 1) / gb > 65535 || M < 1) {
+    auto on_host = [&]() -> int {
         for (int64_t g = 0; g < G; ++g) {
             const int rc = rg_kpm_density(mu + 2 * g * M, M, x, nx, edge_inset, kernel, rho + g * nx);
             if (rc) return fail(ctx, rc, "density reconstruction failed");
         }
         return RG_OK;
-    }
+    };
+    // Few terms stay on the host: a launch with its transfers costs about
+    // 45 us, the host loop 2.2 ns a term.
+    if ((double)G * M * nx < 2e4 || M < 1) return on_host();
     RG_HIP(ctx, hipSetDevice(ctx->device), "hipSetDevice");
-    // weights (2 - delta_m0) g_m Re mu_m packed [block][m][gb], then the grid
-    const int64_t nb = (G + gb - 1) / gb;
-    std::vector<double> in((size_t)(nb * M * gb + nx), 0.0);
-    for (int64_t g = 0; g < G; ++g) {
-        double *o = in.data() + (g / gb) * M * gb + g % gb;
-        const double *m = mu + 2 * g * M;
-        o[0] = gk[0] * m[0];
-        for (int k = 1; k < M; ++k) o[(int64_t)k * gb] = 2.0 * gk[k] * m[2 * k];
-    }
-    std::copy(x, x + nx, in.begin() + (ptrdiff_t)(nb * M * gb));
-    RG_HIP(ctx, ctx->den_in.ensure(in.size() * 8), "hipMalloc density");
-    RG_HIP(ctx, ctx->den_out.ensure((size_t)(G * nx) * 8), "hipMalloc density");
-    RG_HIP(ctx, hipMemcpyAsync(ctx->den_in.p, in.data(), in.size() * 8, hipMemcpyHostToDevice, ctx->stream),
-           "upload density weights");
+    // The grid and the blocks of gb sets are cut so that a piece's weights, grid
+    // and result take about kDensityBytes, whatever the number of sets.
+    constexpr int64_t kDensityBytes = (int64_t)128 << 20, kPoints = (int64_t)1 << 20;
+    const int64_t nxs = std::min(nx, kPoints), nb = (G + gb - 1) / gb;
+    const int64_t nbs = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(nb, 65535), kDensityBytes / (8 * gb * (M + nxs))));
+    std::vector<double> in((size_t)(nbs * M * gb + nxs));
+    if (!store(ctx, ctx->den_in, in.size() * 8) || !store(ctx, ctx->den_out, (size_t)(nbs * gb * nxs) * 8))
+        return on_host();
     const double *w = static_cast<const double *>(ctx->den_in.p);
-    RG_HIP(ctx, launch_density(w, G, M, w + nb * M * gb, nx, edge_inset, static_cast<double *>(ctx->den_out.p),
-                               ctx->stream),
-           "density launch");
-    RG_HIP(ctx, hipMemcpyAsync(rho, ctx->den_out.p, (size_t)(G * nx) * 8, hipMemcpyDeviceToHost, ctx->stream),
-           "download density");
-    RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    for (int64_t j0 = 0; j0 < nx; j0 += nxs)
+        for (int64_t g0 = 0; g0 < G; g0 += nbs * gb) {
+            const int64_t nj = std::min(nxs, nx - j0), ng = std::min(nbs * gb, G - g0), blocks = (ng + gb - 1) / gb;
+            // weights (2 - delta_m0) g_m Re mu_m packed [block][m][gb], then the grid
+            std::fill(in.begin(), in.end(), 0.0);
+            for (int64_t g = 0; g < ng; ++g) {
+                double *o = in.data() + (g / gb) * M * gb + g % gb;
+                const double *m = mu + 2 * (g0 + g) * M;
+                o[0] = gk[0] * m[0];
+                for (int k = 1; k < M; ++k) o[(int64_t)k * gb] = 2.0 * gk[k] * m[2 * k];
+            }
+            std::copy(x + j0, x + j0 + nj, in.begin() + (ptrdiff_t)(blocks * M * gb));
+            RG_HIP(ctx, hipMemcpyAsync(ctx->den_in.p, in.data(), (size_t)(blocks * M * gb + nj) * 8, hipMemcpyHostToDevice,
+                                       ctx->stream),
+                   "upload density weights");
+            RG_HIP(ctx, launch_density(w, ng, gb, M, w + blocks * M * gb, nj, edge_inset,
+                                       static_cast<double *>(ctx->den_out.p), ctx->stream),
+                   "density launch");
+            if (nj == nx)
+                RG_HIP(ctx, hipMemcpyAsync(rho + g0 * nx, ctx->den_out.p, (size_t)(ng * nx) * 8, hipMemcpyDeviceToHost,
+                                           ctx->stream),
+                       "download density");
+            else
+                RG_HIP(ctx, hipMemcpy2DAsync(rho + g0 * nx + j0, (size_t)nx * 8, ctx->den_out.p, (size_t)nj * 8,
+                                             (size_t)nj * 8, (size_t)ng, hipMemcpyDeviceToHost, ctx->stream),
+                       "download density");
+            RG_HIP(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+        }
     return RG_OK;
 }
 

@@ -194,11 +194,11 @@ hipError_t launch_group_finish(int64_t G, const int64_t *grp_chunk, int ndot,
 
 // ---- density reconstruction (rg_density.hip) ----
 // Moment sets one lane evaluates together (1 or 8); the weights of
-// launch_density are packed [ceil(G / batch)][M][batch].
+// launch_density are packed [ceil(G / gb)][M][gb], gb = density_batch.
 int density_batch(int64_t G);
 // rho[g * nx + j] = sum_m w_gm T_m(x_j) / (pi sqrt(max(1e-14, 1 - x_j^2))),
-// x_j clamped to 1 - edge_inset; G <= 65535 * batch
-hipError_t launch_density(const double *w, int64_t G, int M, const double *x, int64_t nx, double edge_inset,
+// x_j clamped to 1 - edge_inset; G <= 65535 gb
+hipError_t launch_density(const double *w, int64_t G, int gb, int M, const double *x, int64_t nx, double edge_inset,
                           double *rho, hipStream_t st);
 
 // ---- graph-local S^{-1/2} patches (rg_isqrt.hip) ----

@@ -64,3 +64,30 @@ def test_projected_run_without_room_for_its_stores(monkeypatch):
         assert np.array_equal(x, y)
     # 4,096 chunks of 48 bytes in each of 257 steps
     assert held[None] - held[str(MB)] > 40 * MB
+
+
+@pytest.mark.parametrize("G,M,nx", [(2100, 3, 20000), (9, 3, (1 << 20) + 7), (1, 2, (1 << 20) + 1)])
+def test_density_takes_bounded_memory(G, M, nx):
+    """Many sets, or a grid above a million points, go through the device in
+    pieces (128 MB, and what an allocation rounds up to)."""
+    rng = np.random.default_rng(G)
+    mu = rng.standard_normal((G, M)) + 1j * rng.standard_normal((G, M))
+    x = np.linspace(-1.01, 1.01, nx)
+    with _lib.Context(0) as ctx:
+        free = ctx.mem_info()[0]
+        rho = ctx.kpm_density(mu, x, 0.5 / nx)
+        assert free - ctx.mem_info()[0] < 160 * MB
+    ref = np.stack([_lib.kpm_density(m, x, 0.5 / nx) for m in mu])
+    assert np.array_equal(rho, ref)
+
+
+def test_density_without_room(monkeypatch):
+    monkeypatch.setenv("RG_STORE_MAX", "1000")
+    rng = np.random.default_rng(4)
+    mu = rng.standard_normal((33, 64)) + 1j * rng.standard_normal((33, 64))
+    x = np.linspace(-1.01, 1.01, 1000)
+    with _lib.Context(0) as ctx:
+        free = ctx.mem_info()[0]
+        rho = ctx.kpm_density(mu, x, 0.5 / 1000)
+        assert ctx.mem_info()[0] == free
+    assert np.array_equal(rho, np.stack([_lib.kpm_density(m, x, 0.5 / 1000) for m in mu]))
