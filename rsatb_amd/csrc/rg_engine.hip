@@ -177,7 +177,7 @@ struct rg_context {
     DevBuf dpart; // per-step dot partials of a run whose reductions are deferred
     // projected moments: rows sorted by group, chunk and group ranges, dots
     DevBuf pd_rows, pd_chunk, pd_grp, pd_partial, pd_out;
-    // dpart and pd_partial hold a run's dots: not to be given back
+    // dpart, pd_partial or kg_part is in use: none is given back
     bool stores_busy = false;
     // bytes a store may take that a call can do without (RG_STORE_MAX)
     size_t store_max = (size_t)1 << 30;
@@ -273,7 +273,8 @@ bool give_back(rg_context *ctx) {
     bool any = ctx->upload_staging.p != nullptr;
     ctx->upload_staging.release();
     if (!ctx->stores_busy) {
-        any = any || ctx->dpart.p || ctx->pd_partial.p;
+        any = any || ctx->dpart.p || ctx->pd_partial.p || ctx->kg_part.p;
+        ctx->kg_part.release();
         ctx->dpart.release();
         ctx->pd_partial.release();
     }
@@ -296,7 +297,7 @@ hipError_t ensure(rg_context *ctx, DevBuf &buf, size_t n) {
 
 // True when buf holds n bytes; false when that is more than a store may take or
 // than there is, and the call does without.
-bool store(rg_context *ctx, DevBuf &buf, size_t n) {
+bool room_for(rg_context *ctx, DevBuf &buf, size_t n) {
     return n <= ctx->store_max && ensure(ctx, buf, n) == hipSuccess;
 }
 
@@ -1178,7 +1179,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     const bool onchip = ctx->onchip && doubled && !keep && !ctx->prof && ctx->form == RG_FORM_ORTHOGONAL &&
                         onchip_fits(dev_view(ctx->slots[RG_SLOT_H], vm.fp32), vm);
     const bool defer = doubled && !onchip && !noalloc && nsteps > 2 &&
-                       store(ctx, ctx->dpart, (size_t)nsteps * (size_t)pstride * 16);
+                       room_for(ctx, ctx->dpart, (size_t)nsteps * (size_t)pstride * 16);
     double2 *dparts = defer ? static_cast<double2 *>(ctx->dpart.p) : nullptr;
     const StoresScope stores(ctx, defer);
 
@@ -1698,7 +1699,7 @@ int rg_kpm_pdos_moments(rg_context *ctx, int M, int precision, int doubling, int
     // a doubled run keeps every step's chunk dots and finishes them in one
     // launch (the same sums in the same order) when there is room for them
     const size_t part_bytes = (size_t)std::max<int64_t>(nchunks, 1) * 3 * 16;
-    const bool defer = doubled && store(ctx, ctx->pd_partial, part_bytes * (size_t)nsteps);
+    const bool defer = doubled && room_for(ctx, ctx->pd_partial, part_bytes * (size_t)nsteps);
     if (!defer) RG_HIP(ctx, ctx->pd_partial.ensure(part_bytes), "hipMalloc group partials");
     RG_HIP(ctx, hipMemcpy(ctx->pd_rows.p, rows.data(), rows.size() * 4, hipMemcpyHostToDevice),
            "upload group rows");
@@ -2379,6 +2380,7 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     double *Qz = Wz + 3 * zmat;
     double *dmud = Qz + 3 * (size_t)np * zmat; // tangent moments (mu_real doubles)
     const double s2 = 1.0 / (4.0 * ha * ha);
+    const StoresScope stores(ctx, true);
     // out[pi] (+)= s^2 Lseq(a)^H Rseq(b) for every pair: real sequences in one
     // launch (k_kg_gemm), complex ones a library product each.
     // Complex FP32 sequences: K is cut into chunks of Kc rows; each chunk of the M
@@ -2394,8 +2396,20 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
         Kc = std::max<size_t>(1, std::min(K, budget / (2 * (size_t)M * 8 * cw)));
         RG_HIP(ctx, ctx->kg_work.ensure(2 * (size_t)M * Kc * 8 * cw), "hipMalloc widening panels");
     }
-    const KgGemmPlan gp = kg_gemm_plan(M, (int64_t)K, np);
-    if (!vm.complex_vec) RG_HIP(ctx, ctx->kg_part.ensure(kg_gemm_bytes(gp, np)), "hipMalloc moment parts");
+    // without room for the parts of all products: fewer chunks of K, then one
+    // product at a time
+    KgGemmPlan gp = kg_gemm_plan(M, (int64_t)K, np);
+    int at_once = np;
+    while (!vm.complex_vec && !room_for(ctx, ctx->kg_part, kg_gemm_bytes(gp, at_once))) {
+        if (gp.nchunk > 1) {
+            kg_gemm_chunks(gp, (int64_t)K, gp.nchunk / 2);
+        } else if (at_once > 1) {
+            at_once = 1;
+        } else {
+            RG_HIP(ctx, ctx->kg_part.ensure(kg_gemm_bytes(gp, 1)), "hipMalloc moment parts");
+            break;
+        }
+    }
     auto timed = [&](int products, auto run) -> int { // run() as one launch of the product class
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
         if (ctx->prof) {
@@ -2426,16 +2440,18 @@ int dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, double pref
     };
     auto moment_gemms = [&](auto Lseq, auto Rseq, double *out, double beta_in) -> int {
         if (!vm.complex_vec) {
-            KgGemm p{};
-            for (int pi = 0; pi < np; ++pi) {
-                p.l[pi] = Lseq(comp_a[pairs[pi]], 0);
-                p.r[pi] = Rseq(comp_b[pairs[pi]], 0);
-            }
             return timed(np, [&]() -> int {
-                RG_HIP(ctx, launch_kg_gemm(gp, p, np, fp32, (int64_t)K, (int64_t)Kp, M, s2, beta_in,
-                                           static_cast<double *>(ctx->kg_part.p), ctx->kg_part.bytes, out, (int64_t)mm,
-                                          ctx->stream),
-                       "moment products");
+                for (int p0 = 0; p0 < np; p0 += at_once) {
+                    KgGemm p{};
+                    for (int q = 0; q < at_once; ++q) {
+                        p.l[q] = Lseq(comp_a[pairs[p0 + q]], 0);
+                        p.r[q] = Rseq(comp_b[pairs[p0 + q]], 0);
+                    }
+                    RG_HIP(ctx, launch_kg_gemm(gp, p, at_once, fp32, (int64_t)K, (int64_t)Kp, M, s2, beta_in,
+                                               static_cast<double *>(ctx->kg_part.p), ctx->kg_part.bytes,
+                                               out + (size_t)p0 * mm, (int64_t)mm, ctx->stream),
+                           "moment products");
+                }
                 return RG_OK;
             });
         }
@@ -3327,7 +3343,7 @@ int rg_kpm_density_batch(rg_context *ctx, const double *mu, int64_t G, int M, co
     const int64_t nxs = std::min(nx, kPoints), nb = (G + gb - 1) / gb;
     const int64_t nbs = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(nb, 65535), kDensityBytes / (8 * gb * (M + nxs))));
     std::vector<double> in((size_t)(nbs * M * gb + nxs));
-    if (!store(ctx, ctx->den_in, in.size() * 8) || !store(ctx, ctx->den_out, (size_t)(nbs * gb * nxs) * 8))
+    if (!room_for(ctx, ctx->den_in, in.size() * 8) || !room_for(ctx, ctx->den_out, (size_t)(nbs * gb * nxs) * 8))
         return on_host();
     const double *w = static_cast<const double *>(ctx->den_in.p);
     for (int64_t j0 = 0; j0 < nx; j0 += nxs)

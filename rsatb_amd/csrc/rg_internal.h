@@ -301,6 +301,7 @@ struct KgGemmPlan {
     int64_t kc = 16;
 };
 KgGemmPlan kg_gemm_plan(int M, int64_t K, int npairs);
+void kg_gemm_chunks(KgGemmPlan &p, int64_t K, int64_t want);
 inline size_t kg_gemm_bytes(const KgGemmPlan &p, int npairs) {
     const size_t side = (size_t)p.nt * 32 * p.a;
     return (size_t)npairs * p.nchunk * side * side * 8;

@@ -400,9 +400,14 @@ KgGemmPlan kg_gemm_plan(int M, int64_t K, int npairs) {
         for (int64_t c = 2; c <= top; ++c) least = std::min(least, time(c));
         for (want = 1; time(want) > 1.05 * least;) ++want;
     }
+    kg_gemm_chunks(p, K, want);
+    return p;
+}
+
+// K in at most `want` chunks of whole blocks of sixteen
+void kg_gemm_chunks(KgGemmPlan &p, int64_t K, int64_t want) {
     p.kc = ((K + want - 1) / want + 15) / 16 * 16;
     p.nchunk = (int)((K + p.kc - 1) / p.kc);
-    return p;
 }
 
 hipError_t launch_kg_gemm(const KgGemmPlan &pl, const KgGemm &p, int npairs, bool fp32, int64_t K, int64_t ld, int M,

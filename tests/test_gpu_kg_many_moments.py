@@ -84,3 +84,22 @@ def test_rate_does_not_fall_with_the_moments():
         return best
 
     assert rate(1500, 4096, 16) >= 0.5 * rate(512, 8192, 16)
+
+
+@pytest.mark.parametrize("formulation", [0, 1])
+@pytest.mark.parametrize("limit", ["0", "100000", "3000000"])
+def test_moments_without_room_for_the_parts(formulation, limit, monkeypatch):
+    """Fewer chunks of K, or one product at a time, give the same exact moments."""
+    n, R, M = 1024, 1, 200
+    rng = np.random.default_rng(8)
+    h, ts, H, V = operators(n, rng)
+    psi = rng.integers(-3, 4, (n, R)).astype(float)
+    with context(n, R, H, V, psi) as ctx:
+        want = ctx.dc_spectrum(M, formulation, with_moments=True)[2]
+        full = ctx.mem_info()[0]
+    monkeypatch.setenv("RG_STORE_MAX", limit)
+    with context(n, R, H, V, psi) as ctx:
+        for prec in (_lib.PREC_FP64, _lib.PREC_FP32):
+            assert np.array_equal(ctx.dc_spectrum(M, formulation, with_moments=True, precision=prec)[2], want)
+        # sixteen chunks of three or six products, 256 x 256 each, take 25 MB or 50
+        assert ctx.mem_info()[0] - full > 16 * (1 << 20)
