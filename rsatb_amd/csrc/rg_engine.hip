@@ -114,20 +114,19 @@ struct Slot {
     bool is_complex = false;
     DevBuf row_ptr, col_ind, vals64, vals32;
     bool vals32_valid = false;
-    // gather table of the MFMA SpMM (see BsrDev): the offsets (xoff_bytes), then
-    // the entries
+    // gather table of the MFMA SpMM (see BsrDev)
     DevBuf xrow;
     int64_t xlen = 0;
     bool has_xrow = false;
     // The MFMA SpMM's own view of the slot (real, b >= 8): block rows in a
-    // processing order of compact regions of sreg rows (sched), and every
+    // processing order of compact regions of sreg rows, and every
     // row's blocks in the order of a distance-2 colouring of the block
     // columns (kperm: the stored block behind every position; kcol and kxrow
     // the column indices and gather table in that order). The values in that
     // order (kvals64, kvals32) are copies remade after a write of the slot:
     // they are current when their generation equals gen.
     bool has_plan = false;
-    DevBuf sched, kperm, kcol, kxrow, kvals64, kvals32;
+    DevBuf kperm, kcol, kxrow, kvals64, kvals32;
     uint64_t kvals64_gen = 0, kvals32_gen = 0;
     // blocks in every block row when they are all equal (0: ragged)
     int32_t ulen = 0;
@@ -346,9 +345,6 @@ bool vec_complex(const rg_context *ctx) {
 
 size_t vec_elem_bytes(VecMode vm) { return (vm.complex_vec ? 2 : 1) * (vm.fp32 ? 4 : 8); }
 
-// Bytes of a gather table's offsets, in whole 16-byte pieces.
-size_t xoff_bytes(int64_t nbr) { return ((size_t)nbr + 2) / 2 * 16; }
-
 // True when the slot's MFMA view (the scheduled rows and colour-ordered
 // blocks) holds current values for the precision.
 bool plan_current(const Slot &s, bool fp32) {
@@ -368,15 +364,13 @@ BsrDev dev_view(const Slot &s, bool fp32) {
     d.ulen = s.ulen;
     d.maxlen = s.maxlen;
     auto table = [&](const DevBuf &t) {
-        d.xoff = static_cast<const int64_t *>(t.p);
-        d.xrow = reinterpret_cast<const int32_t *>(static_cast<const char *>(t.p) + xoff_bytes(s.nbr));
+        d.mrow = static_cast<const MfmaRow *>(t.p);
         d.xlen = s.xlen;
     };
     if (plan_current(s, fp32)) {
         d.col_ind = static_cast<const int32_t *>(s.kcol.p);
         d.vals = fp32 ? s.kvals32.p : s.kvals64.p;
         table(s.kxrow);
-        d.sched = static_cast<const int32_t *>(s.sched.p);
         return d;
     }
     d.col_ind = static_cast<const int32_t *>(s.col_ind.p);
@@ -579,9 +573,9 @@ MfmaPlan mfma_plan(int64_t n, const int64_t *rp, const int32_t *ci, int32_t sreg
     return pl;
 }
 
-// Gather table (see BsrDev::xrow) of a slot with b >= 8, the blocks the MFMA
-// SpMM takes, and the plan of a real one; kXrowSpare trailing entries keep the steps it fetches past
-// the last row's K in range.
+// Gather table (see BsrDev::mrow) of a slot with b >= 8, the blocks the MFMA
+// SpMM takes, and the plan of a real one; kXrowSpare trailing entries keep the
+// steps it fetches past the last row's K in range.
 int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     s.has_xrow = false;
     s.has_plan = false;
@@ -598,22 +592,31 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     if ((int64_t)s.nbr * s.b > INT32_MAX) return RG_OK;
     // A ragged last step repeats the row's last X row: its A elements are zero,
     // and another row's X could hold an infinity, which zero does not cancel.
-    auto steps4 = [&](int64_t r) { return ((rp[r + 1] - rp[r]) * s.b + 3) / 4 * 4; };
+    const int b = s.b;
+    auto steps4 = [&](int64_t r) { return ((rp[r + 1] - rp[r]) * b + 3) / 4 * 4; };
     s.xlen = 0;
     for (int64_t r = 0; r < s.nbr; ++r) s.xlen += steps4(r);
-    const size_t head = xoff_bytes(s.nbr) / 4; // of the offsets, in entries
+    if (s.nnzb > INT32_MAX || s.xlen / 4 > UINT32_MAX) return RG_OK;
+    const size_t head = 4 * (size_t)s.nbr; // of the rows, in entries
     std::vector<int32_t> t(head + (size_t)s.xlen + kXrowSpare, 0);
     auto fill = [&](const int32_t *cols, const int32_t *order) {
-        int32_t *o = t.data() + head;
+        int32_t *const first = t.data() + head;
         int64_t at = 0;
         for (int64_t p = 0; p < s.nbr; ++p) {
-            std::memcpy(t.data() + 2 * p, &at, 8);
             const int64_t r = order ? order[p] : p;
+            const MfmaRow row{(uint32_t)(at / 4), (int32_t)rp[r], (int32_t)(rp[r + 1] - rp[r]), (int32_t)r};
+            std::memcpy(t.data() + 4 * p, &row, sizeof(row));
+            int32_t *o = first + at;
+            // sixteen entries a block at once: what lies past its b is written again,
+            // or a spare one
+            for (int64_t q = rp[r]; q < rp[r + 1]; ++q, o += b) {
+                const int32_t x0 = cols[q] * b;
+                for (int kk = 0; kk < 16; ++kk) o[kk] = x0 + kk;
+            }
             at += steps4(r);
-            for (int64_t q = rp[r]; q < rp[r + 1]; ++q)
-                for (int kk = 0; kk < s.b; ++kk) *o++ = cols[q] * s.b + kk;
-            for (; o < t.data() + head + at; ++o) *o = o[-1];
+            for (; o < first + at; ++o) *o = o[-1];
         }
+        std::fill(first + at, first + at + kXrowSpare, 0);
     };
     fill(ci, nullptr);
     RG_HIP(ctx, s.xrow.ensure(t.size() * 4), "hipMalloc gather table");
@@ -625,11 +628,9 @@ int build_xrow(rg_context *ctx, Slot &s, const int64_t *rp, const int32_t *ci) {
     std::vector<int32_t> kc((size_t)s.nnzb + 1, 0);
     for (int64_t q = 0; q < s.nnzb; ++q) kc[(size_t)q] = ci[pl.kperm[(size_t)q]];
     fill(kc.data(), pl.sched.data());
-    RG_HIP(ctx, s.sched.ensure((size_t)s.nbr * 4), "hipMalloc row schedule");
     RG_HIP(ctx, s.kperm.ensure((size_t)s.nnzb * 4 + 4), "hipMalloc block order");
     RG_HIP(ctx, s.kcol.ensure(kc.size() * 4), "hipMalloc block order");
     RG_HIP(ctx, s.kxrow.ensure(t.size() * 4), "hipMalloc gather table");
-    RG_HIP(ctx, hipMemcpy(s.sched.p, pl.sched.data(), (size_t)s.nbr * 4, hipMemcpyHostToDevice), "upload plan");
     if (s.nnzb > 0)
         RG_HIP(ctx, hipMemcpy(s.kperm.p, pl.kperm.data(), (size_t)s.nnzb * 4, hipMemcpyHostToDevice),
                "upload plan");
@@ -654,10 +655,9 @@ int copy_tables(rg_context *ctx, Slot &d, const Slot &src) {
     d.has_xrow = d.has_plan = false;
     d.kvals64_gen = d.kvals32_gen = 0;
     d.xlen = src.xlen;
-    const size_t nt = xoff_bytes(src.nbr) + ((size_t)src.xlen + kXrowSpare) * 4;
+    const size_t nt = (size_t)src.nbr * sizeof(MfmaRow) + ((size_t)src.xlen + kXrowSpare) * 4;
     if (src.has_xrow) RG_HIP(ctx, copy(d.xrow, src.xrow, nt), "copy gather table");
     if (src.has_plan) {
-        RG_HIP(ctx, copy(d.sched, src.sched, (size_t)src.nbr * 4), "copy plan");
         RG_HIP(ctx, copy(d.kperm, src.kperm, (size_t)src.nnzb * 4 + 4), "copy plan");
         RG_HIP(ctx, copy(d.kcol, src.kcol, (size_t)src.nnzb * 4 + 4), "copy plan");
         RG_HIP(ctx, copy(d.kxrow, src.kxrow, nt), "copy plan");
@@ -1261,7 +1261,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
         for (void *w : wv) key.push_back(addr(w));
         for (int sl = 0; sl < (ctx->form == RG_FORM_SANDWICH ? 3 : 1); ++sl) {
             const BsrDev q = dev_view(ctx->slots[sl], vm.fp32);
-            for (uint64_t x : {addr(q.row_ptr), addr(q.col_ind), addr(q.vals), addr(q.xrow), addr(q.xoff), addr(q.sched),
+            for (uint64_t x : {addr(q.row_ptr), addr(q.col_ind), addr(q.vals), addr(q.mrow),
                                (uint64_t)q.ulen, (uint64_t)q.nbr, (uint64_t)q.b, (uint64_t)q.nnzb,
                                (uint64_t)q.is_complex})
                 key.push_back(x);

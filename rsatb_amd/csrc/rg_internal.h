@@ -11,6 +11,13 @@ namespace rg {
 // step after its last fetch (PD <= 8: 8 PD - 4 = 60 entries).
 constexpr int kXrowSpare = 64;
 
+// One block row as the MFMA SpMM processes it: block row br with blocks s0 ..
+// s0 + nblk - 1, its X rows from entry 4 at4 of the gather table on.
+struct MfmaRow {
+    uint32_t at4;
+    int32_t s0, nblk, br;
+};
+
 // Device view of one BSR operand. Values are real (vals) or complex
 // interleaved (vals with is_complex), in double or float storage.
 struct BsrDev {
@@ -21,16 +28,12 @@ struct BsrDev {
     const int32_t *col_ind = nullptr;
     const void *vals = nullptr; // double / double2 / float / float2
     bool is_complex = false;
-    // gather table of b >= 8 matrices, or null: from xoff[p] on the X rows
-    // (col_ind[s] * b + kk of block s, column kk) of the columns of the block row
-    // at position p, in whole steps of four (a ragged last step repeats the row's
+    // gather table of b >= 8 matrices, or null: the nbr block rows in processing
+    // order, then int32 entries, every row's X rows (col_ind[s] * b + kk of block
+    // s, column kk) in whole steps of four (a ragged last step repeats the row's
     // last X row); xlen entries in all, then kXrowSpare spare ones
-    const int32_t *xrow = nullptr;
-    const int64_t *xoff = nullptr;
+    const MfmaRow *mrow = nullptr;
     int64_t xlen = 0;
-    // processing order of the block rows (MFMA SpMM), or null for stored
-    // order: position p of [0, nbr) computes block row sched[p]
-    const int32_t *sched = nullptr;
     // > 0 when every block row holds exactly ulen blocks and row_ptr[0] = 0:
     // row br's blocks are then br * ulen .. br * ulen + ulen - 1, and the VALU
     // SpMM computes them instead of loading row_ptr

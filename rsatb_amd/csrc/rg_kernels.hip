@@ -995,7 +995,7 @@ static int valu_launch_grid(const BsrDev &A, VecMode vm, int R) {
 static MfmaShape mfma_shape(const BsrDev &A, bool fp32, bool cv, int R) {
     MfmaShape s;
     const int W = R * (cv ? 2 : 1);
-    if (A.b < 8 || !A.xrow || (A.is_complex && !cv) || W > 512) return s;
+    if (A.b < 8 || !A.mrow || (A.is_complex && !cv) || W > 512) return s;
     s.nchunks = W > 256 ? 2 : 1;
     const int per = (W + s.nchunks - 1) / s.nchunks; // columns a chunk must hold
     static const int even64[] = {2, 4, 6, 8, 12, 16}, even32[] = {2, 4, 8, 12, 16}, half32[] = {2, 4, 8, 16};

@@ -384,14 +384,12 @@ template <typename S, int NT, int MODE, bool CV, bool CM> constexpr int prefetch
 // W = 256 216 -> 205, 236 -> 223 and 290 -> 253 us (first).
 template <typename S, int NT, int E, bool MASK, int MODE, bool CV, bool CM>
 __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spmm_mfma(int64_t nbr, int b,
-                                                   const int64_t *__restrict__ row_ptr,
-                                                   const int64_t *__restrict__ xoff,
+                                                   const MfmaRow *__restrict__ rows,
                                                    const int32_t *__restrict__ xrow,
                                                    const S *__restrict__ vals,
                                                    const S *__restrict__ zero,
                                                    const S *__restrict__ X, S *__restrict__ Y,
                                                    int W, int R, int nchunks, int xcd_map,
-                                                   const int32_t *__restrict__ sched,
                                                    EpiArgs e) {
     using A4 = typename Acc4<S>::T;
     typedef S A2 __attribute__((ext_vector_type(2)));
@@ -417,7 +415,7 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
     // XCD walks its own contiguous eighth of the block rows, so the rows in
     // flight on one XCD (and their gathered neighbours) stay close together
     // in its L2.
-    // Position p computes block row sched[p]; the eighths are cut by rows, not
+    // Position p computes block row rows[p].br; the eighths are cut by rows, not
     // by whole regions: an operator of ten regions gave two XCDs twice the
     // rows of the others.
     int64_t r_lo = 0, r_hi = nbr;
@@ -441,9 +439,11 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
     const int32_t m0 = g == 0 ? -1 : 0, m1 = g == 1 ? -1 : 0, m2 = g == 2 ? -1 : 0, m3 = g == 3 ? -1 : 0;
     for (int64_t it = kq * kMfmaWaves + wave; it < total; it += nk * kMfmaWaves) {
         const int64_t pos = r_lo + it / nchunks;
-        const int64_t br = sched ? (int64_t)sched[pos] : pos;
-        const int64_t s0 = row_ptr[br];
-        const int nblk = (int)(row_ptr[br + 1] - s0);
+        // one 16-byte scalar load: a row's chain is this, the table, the gathers
+        const MfmaRow row = rows[pos];
+        const int64_t br = row.br, s0 = row.s0;
+        const int nblk = row.nblk;
+        int64_t kb = (int64_t)row.at4 * 4;
         const int nsteps = (nblk * b + 3) >> 2;
         // the first output rows' Xs, Xp values, in flight during the K loop
         S pxs[NT], pxp[NT];
@@ -470,7 +470,6 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
         const int K = nblk * b;
         const AT *__restrict__ panel = reinterpret_cast<const AT *>(vals) + s0 * (int64_t)b * b;
         int fst = 0; // next step to fetch
-        int64_t kb = xoff[pos];
         int32_t nx0 = xrow[kb], nx1 = xrow[kb + 1], nx2 = xrow[kb + 2], nx3 = xrow[kb + 3];
         auto fetch = [&](AT &a, S (&bv)[NT]) {
             // masks, not a select: the compiler branched over the lane groups
@@ -562,15 +561,13 @@ hipError_t go_mfma(const MfmaShape &s, const BsrDev &A, const void *X, void *Y, 
     const int grid = std::min(grid_req, g_mfma.grid_cap > 0 ? g_mfma.grid_cap : res);
     if (grid_out) *grid_out = grid;
     if (t_mfma_grid_query) return hipSuccess;
-    // the zero element of lanes outside a panel: row_ptr[0] (0, checked when
-    // a slot is written) for real values; for complex ones 16 aligned zero
-    // bytes of the gather table's spare entries
-    const void *zero = CM ? static_cast<const void *>(A.xrow + A.xlen)
-                          : static_cast<const void *>(A.row_ptr);
+    // the zero element of lanes outside a panel: 16 aligned zero bytes of the
+    // gather table's spare entries
+    const int32_t *xrow = reinterpret_cast<const int32_t *>(A.mrow + A.nbr);
+    const void *zero = xrow + A.xlen;
     hipLaunchKernelGGL((k_spmm_mfma<S, NT, E, MASK, MODE, CV, CM>), dim3(grid), dim3(64 * kMfmaWaves), 0, st, A.nbr,
-                       (int)A.b, A.row_ptr, A.xoff, A.xrow, static_cast<const S *>(A.vals), static_cast<const S *>(zero),
-                       static_cast<const S *>(X), static_cast<S *>(Y), W, R, s.nchunks, g_mfma.xcd_map, A.sched,
-                       e);
+                       (int)A.b, A.mrow, xrow, static_cast<const S *>(A.vals), static_cast<const S *>(zero),
+                       static_cast<const S *>(X), static_cast<S *>(Y), W, R, s.nchunks, g_mfma.xcd_map, e);
     return hipGetLastError();
 }
 
