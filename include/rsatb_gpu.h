@@ -362,8 +362,8 @@ RG_API int rg_dc_spectrum(rg_context *ctx, int M, int formulation, int kernel, d
 
 /* rg_dc_spectrum with a precision (RG_PREC_FP64 or RG_PREC_FP32). FP32: the
  * recurrence and the velocity products run on FP32 vectors and matrices and
- * the stored sequences are FP32 (half the memory); the moment GEMMs widen
- * K-chunks of them to FP64 and accumulate in FP64. The reference's transport
+ * the stored sequences are FP32 (half the memory); the moment products
+ * widen them to FP64 (exactly) and accumulate in FP64. The reference's transport
  * path is FP64 only (dc_spectrum_fftcheb, fftcheb_transport.hpp:543-653);
  * this is the precision form of that spectrum. */
 RG_API int rg_dc_spectrum_ex(rg_context *ctx, int M, int formulation, int kernel, double prefactor, int precision,
@@ -413,7 +413,11 @@ RG_API int rg_cancel(rg_context *ctx);
 
 /* ---- measurement (no reference counterpart; for the benchmark) ---- */
 
-/* Turns per-launch HIP event timing on (1) or off (0) and clears stats. */
+/* Turns per-launch HIP event timing on (1) or off (0) and clears stats. While
+ * it is on, what else goes in one launch is launched step by step (the moment
+ * loop of small scalar operators, the conductivity sequences): the vectors are
+ * the same, the moments of those small operators differ by the order of their
+ * sums (FP64 rounding). */
 RG_API int rg_set_profiling(rg_context *ctx, int on);
 
 /* Kernel classes timed when profiling is on. */
