@@ -373,6 +373,7 @@ template <typename S, bool CM, bool CV>
 hipError_t by_block(const BsrDev &A, const void *X, void *Y, int R, const EpiArgs &e, int grid,
                     hipStream_t st) {
     if (A.b == 1) return by_layout<S, CM, CV, 1>(A, X, Y, R, e, grid, st);
+    if (A.b == 13) return by_layout<S, CM, CV, 13>(A, X, Y, R, e, grid, st);
     return by_layout<S, CM, CV, 0>(A, X, Y, R, e, grid, st);
 }
 
@@ -982,6 +983,15 @@ static int valu_launch_grid(const BsrDev &A, VecMode vm, int R) {
         }
     const int g = valu_grid(A.nbr, valu_lpr(A, vm.fp32, vm.complex_vec, R));
     return b1v_lpr(A, vm.fp32, vm.complex_vec, R) ? (g + 7) / 8 * 8 : g;
+}
+
+int spmm_grid(int64_t nbr, int R) {
+    const int G = 64 / lpr_for(R);
+    const int64_t rows_per_wg = (int64_t)kWaves * G;
+    int64_t g = (nbr + rows_per_wg - 1) / rows_per_wg;
+    if (g > kMaxGrid) g = kMaxGrid;
+    if (g < 1) g = 1;
+    return (int)g;
 }
 
 // The MFMA launch shape for this operand, or nt = 0 when it takes the VALU
