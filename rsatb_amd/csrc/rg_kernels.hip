@@ -1009,9 +1009,9 @@ static MfmaShape mfma_shape(const BsrDev &A, bool fp32, bool cv, int R) {
     s.nchunks = W > 256 ? 2 : 1;
     const int per = (W + s.nchunks - 1) / s.nchunks; // columns a chunk must hold
     static const int even64[] = {2, 4, 6, 8, 12, 16}, even32[] = {2, 4, 8, 12, 16}, half32[] = {2, 4, 8, 16};
-    static const int odd[] = {1, 4, 16};
+    static const int odd[] = {1, 4};
     const int *set = odd;
-    int n = 3;
+    int n = 2;
     s.e = 1;
     if (W % 2 == 0 && (cv || W > 16)) {
         s.e = fp32 && W % 4 == 0 ? 4 : 2;
@@ -1021,6 +1021,8 @@ static MfmaShape mfma_shape(const BsrDev &A, bool fp32, bool cv, int R) {
     int k = 0;
     while (k + 1 < n && 16 * set[k] < per) ++k;
     s.nt = set[k];
+    if (s.e == 1) // odd widths past 64: two or four waves of four tiles, not sixteen tiles mostly empty
+        while (64 * s.nchunks < W && s.nchunks < kWaves) s.nchunks *= 2;
     if (s.nt == 2) s.e = 2; // two tiles hold one 8-byte (FP32) or 16-byte (FP64) access a lane
     if (16 * s.nt * s.nchunks < W) return MfmaShape{};
     const bool pow2 = (s.nt & (s.nt - 1)) == 0;

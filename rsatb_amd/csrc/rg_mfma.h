@@ -611,7 +611,6 @@ hipError_t by_shape(const MfmaShape &s, const BsrDev &A, const void *X, void *Y,
         RG_MFMA_CASE(1, 1, false)
         RG_MFMA_CASE(1, 1, true)
         RG_MFMA_CASE(4, 1, true)
-        RG_MFMA_CASE(16, 1, true)
     }
 #undef RG_MFMA_CASE
     return hipErrorInvalidValue;
