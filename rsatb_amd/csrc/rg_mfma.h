@@ -509,7 +509,43 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
         // unconditional (up to 2 PD - 2 steps past the row: their A lanes read
         // the zero word and their X rows are valid), so the wait before each
         // MFMA group counts only the later buffers' loads on every path.
-        if (nsteps > 0) {
+        if constexpr (PD >= 4) {
+            // Deep buffers stop at the row's end: running on, as below, would fetch
+            // up to 2 PD - 2 steps of nothing, four times the loads of a row of one
+            // block (20,000 rows of a block of 9, one column, FP64, 28.9 -> 15 us; 640
+            // rows of seventeen, W = 16, 9.2 -> 8.5; W = 48 13.2 -> 12.3; W = 40, 1,596
+            // rows of 13, 24.0 -> 24.6).
+            AT ab[PD];
+            S bb[PD][NT];
+            if (nsteps >= PD) {
+#pragma unroll
+                for (int q = 0; q < PD - 1; ++q) fetch(ab[q], bb[q]);
+                int st = 0;
+                for (; st + 2 * PD - 1 <= nsteps; st += PD) {
+#pragma unroll
+                    for (int q = 0; q < PD; ++q) {
+                        fetch(ab[(q + PD - 1) % PD], bb[(q + PD - 1) % PD]);
+                        mma(ab[q], bb[q]);
+                    }
+                }
+                // PD - 1 steps are in flight, up to PD - 1 more to come
+#pragma unroll
+                for (int q = 0; q < PD; ++q) {
+                    if (st + q + PD - 1 < nsteps) fetch(ab[(q + PD - 1) % PD], bb[(q + PD - 1) % PD]);
+                    if (q < PD - 1 || st + q < nsteps) mma(ab[q], bb[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < PD - 2; ++q)
+                    if (st + PD + q < nsteps) mma(ab[q], bb[q]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < PD - 1; ++q)
+                    if (q < nsteps) fetch(ab[q], bb[q]);
+#pragma unroll
+                for (int q = 0; q < PD - 1; ++q)
+                    if (q < nsteps) mma(ab[q], bb[q]);
+            }
+        } else if (nsteps > 0) {
             AT ab[PD];
             S bb[PD][NT];
 #pragma unroll

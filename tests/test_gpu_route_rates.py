@@ -44,3 +44,8 @@ def test_odd_widths_past_64():
     """65 columns take at most 1.5 times the time of 100."""
     H = neighbours(20000, 9, 0)
     assert step_us(H, 65) <= 1.5 * step_us(H, 100)
+
+
+def test_short_rows_do_not_pay_for_deep_buffers():
+    """A block of 9 a row reads a third of what three blocks do."""
+    assert step_us(neighbours(20000, 9, 0), 1) <= 0.8 * step_us(neighbours(20000, 9, 1), 1)
