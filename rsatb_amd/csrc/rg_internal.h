@@ -76,16 +76,14 @@ struct VecMode {
     bool fp32 = false;        // float storage (precision form)
 };
 
-// Number of workgroups the block-row-gather (VALU) SpMM uses for nbr block
-// rows and R columns; spmm_max_grid() bounds every SpMM launch's grid (the
-// dot-partial buffer is sized by it).
-int spmm_grid(int64_t nbr, int R);
+// Bound on every SpMM launch's grid (the dot-partial buffer is sized by it).
 int spmm_max_grid();
 // XCD-contiguous row ranges in the MFMA SpMM (default on).
 void set_xcd_map(int on);
 void set_mfma_ntcap(int nt);
 // cap on the MFMA SpMM's workgroups (a multiple of 8, <= spmm_max_grid());
-// anything else: two workgroups per compute unit (the default)
+// anything else: what is resident, two workgroups per compute unit from eight
+// tiles on and four below (the default)
 void set_mfma_grid_cap(int g);
 void set_b1_wide(int mode);
 void set_uniform_rows(int on);

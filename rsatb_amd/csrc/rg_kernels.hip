@@ -985,13 +985,25 @@ static int valu_launch_grid(const BsrDev &A, VecMode vm, int R) {
     return b1v_lpr(A, vm.fp32, vm.complex_vec, R) ? (g + 7) / 8 * 8 : g;
 }
 
-int spmm_grid(int64_t nbr, int R) {
-    const int G = 64 / lpr_for(R);
-    const int64_t rows_per_wg = (int64_t)kWaves * G;
-    int64_t g = (nbr + rows_per_wg - 1) / rows_per_wg;
-    if (g > kMaxGrid) g = kMaxGrid;
-    if (g < 1) g = 1;
-    return (int)g;
+// Whether few columns on many short rows stay with the VALU kernel, whose waves take
+// eight rows where an MFMA wave (4,096 fit the chip) takes one and pays a row's
+// chain of loads for little. Measured, us a step, MFMA / VALU: FP32, a block of 13 a
+// row, R = 4: 4,000 rows 8.4 / 7.8, 8,000 11.9 / 8.2, 20,000 25.6 / 16.6; five blocks of
+// 13, 8,000 rows 19.6 / 16.4, 20,000 39.9 / 33.8, seventeen, 14,000 rows 68 / 59 (FP64 no
+// slower; a lane sums the dots of a row or two, where compensation gains nothing); a
+// block of 8, 20,000 rows 19.5 / 14.1, 6,000 8.9 / 11.5, of 9 21.1 / 17.5, of 12 20.3 /
+// 21.6; FP64, a block of 13, 8,000 rows 13.5 / 11.9, complex vectors 13.4 / 14.0; a
+// block of 8, 60,000 rows 54.8 / 43.8.
+static bool valu_rows(const BsrDev &A, bool fp32, bool cv, int R) {
+    if (A.nbr < 3500 || R > 16) return false;
+    const int64_t k = A.nnzb * A.b / A.nbr; // columns of an average row's panel
+    const bool one = k <= 13;               // about a block a row
+    if (A.is_complex) return fp32 && one && R <= 8 && (A.b == 13 ? A.nbr >= 6000 : A.b == 8 && A.nbr >= 12000);
+    if (!fp32) return one && !cv && R <= 8 && (A.b == 13 ? A.nbr >= 6000 : A.b == 8 && A.nbr >= 12000);
+    if (A.b == 13) return one || (R <= 8 && A.nbr >= 6000);
+    if (A.nbr < 12000) return false;
+    if (A.b == 8) return one || (k <= 24 && R <= 8);
+    return one && R <= (A.nbr >= 40000 ? 8 : 4) && (A.b <= 10 || (cv && A.b <= 12));
 }
 
 // The MFMA launch shape for this operand, or nt = 0 when it takes the VALU
@@ -1005,7 +1017,7 @@ int spmm_grid(int64_t nbr, int R) {
 static MfmaShape mfma_shape(const BsrDev &A, bool fp32, bool cv, int R) {
     MfmaShape s;
     const int W = R * (cv ? 2 : 1);
-    if (A.b < 8 || !A.mrow || (A.is_complex && !cv) || W > 512) return s;
+    if (A.b < 8 || !A.mrow || (A.is_complex && !cv) || W > 512 || valu_rows(A, fp32, cv, R)) return s;
     s.nchunks = W > 256 ? 2 : 1;
     const int per = (W + s.nchunks - 1) / s.nchunks; // columns a chunk must hold
     static const int even64[] = {2, 4, 6, 8, 12, 16}, even32[] = {2, 4, 8, 12, 16}, half32[] = {2, 4, 8, 16};

@@ -7,8 +7,34 @@ import pytest
 
 from rsatb_amd import _lib
 from rsatb_amd.bsr import BSR
+from test_gpu_mfma_exact import WINDOW, check, exact_columns
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nbr", [5999, 6000])
+def test_exact_on_both_sides_of_the_short_row_rule(oracle, nbr):
+    """Blocks of 13 with few columns: the MFMA kernel below 6,000 block rows, the
+    VALU kernel from there on in FP32 to eight columns."""
+    check(oracle, nbr, 13, False, [1, 8, 9], [1, 8, 9])
+
+
+@pytest.mark.parametrize("b,nbr", [(8, 12000), (9, 12000), (13, 3500), (13, 6000)])
+def test_exact_with_a_block_a_row(oracle, b, nbr):
+    rng = np.random.default_rng(b)
+    d = np.triu(rng.integers(-1, 2, (nbr, b, b)).astype(float))
+    d = d + np.swapaxes(np.triu(d, 1), 1, 2)
+    k = np.arange(nbr)
+    H = BSR.from_blocks(nbr, b, k, k, d)
+    with _lib.Context(0) as ctx:
+        ctx.upload_bsr(_lib.SLOT_H, H)
+        ctx.set_operator(_lib.FORM_ORTHOGONAL, 0.0, WINDOW)
+        for R in (1, 4, 8, 16, 17):
+            psi = rng.choice([-1.0, 1.0], (H.n_rows, R))
+            ctx.set_samples(H.n_rows, R, _lib.SAMPLES_UPLOAD_REAL, data=psi)
+            want = exact_columns(oracle, H, psi, 6, True)
+            for prec in (_lib.PREC_FP64, _lib.PREC_FP32):
+                assert np.array_equal(ctx.kpm_moments(6, precision=prec, per_column=True)[1], want), (R, prec)
 
 
 def neighbours(n, b, width):
@@ -49,3 +75,9 @@ def test_odd_widths_past_64():
 def test_short_rows_do_not_pay_for_deep_buffers():
     """A block of 9 a row reads a third of what three blocks do."""
     assert step_us(neighbours(20000, 9, 0), 1) <= 0.8 * step_us(neighbours(20000, 9, 1), 1)
+
+
+def test_few_fp32_columns_on_many_short_rows():
+    """Half the bytes of FP64, in at most 0.8 of the time."""
+    H = neighbours(20000, 13, 0)
+    assert step_us(H, 4, _lib.PREC_FP32) <= 0.8 * step_us(H, 4)
