@@ -743,6 +743,17 @@ int b1g_cpr(const BsrDev &A, bool fp32, bool cv, int R) {
     const int bytes = R * (fp32 ? 4 : 8) * (cv ? 2 : 1);
     if (bytes % 16 != 0 || bytes / 16 > 256) return 0;
     const int cpr = bytes / 16;
+    // One or two lanes a row read their own long stretches of entries, a cache line a
+    // lane, where a column per lane reads a row's entries once for all its lanes.
+    // Measured at 200,000 rows, column per lane / slab: one lane, FP64, thirteen
+    // entries 26.3 / 15.4 us, seventeen 32.5 / 33.7, twenty-three 42.2 / 60.4; FP32
+    // seventeen 23.9 / 15.8, twenty-three 31.8 / 35.3; two lanes, FP64, seventeen 33.8 /
+    // 26.3, twenty-three 43.5 / 46.0, FP32 twenty-three 34.2 / 31.0, thirty-three 48.2 /
+    // 61.8. The fewer rows in flight, the longer they may be (59,000 rows, two lanes,
+    // forty-nine entries 0.55 to 0.7 of the time; 130,000 rows, one lane, thirty-three
+    // 1.1 to 1.2).
+    const int64_t most = cpr == 1 ? (fp32 ? 19 : 15) : cpr == 2 ? (fp32 ? 27 : 19) : INT32_MAX;
+    if (A.nbr > 100000 && A.nnzb > most * A.nbr) return 0;
     const int64_t g = (A.nbr + 256 / cpr - 1) / (256 / cpr);
     const bool longrow = g_b1g_min_grid > 0 && A.nnzb >= kLongRow * A.nbr;
     return g >= (longrow ? std::min(g_b1g_min_grid, kLongRowMinGrid) : g_b1g_min_grid) ? cpr : 0;

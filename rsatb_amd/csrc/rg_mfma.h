@@ -512,7 +512,7 @@ __global__ __launch_bounds__(256, (sizeof(S) == 8 && NT > 8) ? 1 : 2) void k_spm
         if constexpr (PD >= 4) {
             // Deep buffers stop at the row's end: running on, as below, would fetch
             // up to 2 PD - 2 steps of nothing, four times the loads of a row of one
-            // block (20,000 rows of a block of 9, one column, FP64, 28.9 -> 15 us; 640
+            // block (20,000 rows of a block of 9, one column, FP64, 28.9 -> 17.0 us; 640
             // rows of seventeen, W = 16, 9.2 -> 8.5; W = 48 13.2 -> 12.3; W = 40, 1,596
             // rows of 13, 24.0 -> 24.6).
             AT ab[PD];

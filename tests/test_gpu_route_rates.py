@@ -67,9 +67,10 @@ def step_us(H, R, prec=_lib.PREC_FP64):
 
 
 def test_odd_widths_past_64():
-    """65 columns take at most 1.5 times the time of 100."""
+    """65 columns take at most 1.57 times the time of 100 (1.43 as four waves of four
+    tiles, 1.72 as sixteen tiles)."""
     H = neighbours(20000, 9, 0)
-    assert step_us(H, 65) <= 1.5 * step_us(H, 100)
+    assert step_us(H, 65) <= 1.57 * step_us(H, 100)
 
 
 def test_short_rows_do_not_pay_for_deep_buffers():
@@ -81,3 +82,15 @@ def test_few_fp32_columns_on_many_short_rows():
     """Half the bytes of FP64, in at most 0.8 of the time."""
     H = neighbours(20000, 13, 0)
     assert step_us(H, 4, _lib.PREC_FP32) <= 0.8 * step_us(H, 4)
+
+
+def test_long_rows_of_one_lane(monkeypatch):
+    """Twenty-three entries a row, 16 bytes wide, against the column-per-lane layout."""
+    H = neighbours(200000, 1, 11)
+    slab = step_us(H, 2)
+    monkeypatch.setenv("RG_B1V", "0")
+    plain = step_us(H, 2)
+    monkeypatch.setenv("RG_B1V", "-1")
+    with _lib.Context(0):
+        pass  # the layout knob is the library's: back to its default
+    assert slab <= 1.15 * plain
