@@ -1179,7 +1179,7 @@ int kpm_run(rg_context *ctx, int M, int precision, int doubling, double *mu_out,
     // / so: 336 rows of three 4.2 / 2.2 ms, 1,600 rows of thirteen 4.5 / 3.6, 8,000
     // rows of three 6.1 / 5.7).
     const bool onchip = ctx->onchip && doubled && !keep && !ctx->prof && ctx->form == RG_FORM_ORTHOGONAL &&
-                        onchip_fits(dev_view(ctx->slots[RG_SLOT_H], vm.fp32), vm);
+                        onchip_fits(dev_view(ctx->slots[RG_SLOT_H], vm.fp32), vm, R);
     const bool defer = doubled && !onchip && !noalloc && nsteps > 2 &&
                        room_for(ctx, ctx->dpart, (size_t)nsteps * (size_t)pstride * 16);
     double2 *dparts = defer ? static_cast<double2 *>(ctx->dpart.p) : nullptr;

@@ -171,7 +171,7 @@ struct OnchipWindow {
     double alpha1, beta1, alpha, beta;
 };
 // b = 1, real matrix, few rows: every column's loop runs in one workgroup
-bool onchip_fits(const BsrDev &A, VecMode vm);
+bool onchip_fits(const BsrDev &A, VecMode vm, int R);
 // `steps` doubled steps in one launch. first: t0 holds the samples, and step 0
 // (t1, <0|0>, <0|1>, <1|1>) comes first; else t0, t1 the state of the launch
 // before. The new state is left in t0, t1 ([rows][R] in the storage of vm);

@@ -299,23 +299,32 @@ void onchip_shape(int n, int *rpt, int *nt) {
 
 } // namespace
 
-// Two columns in LDS (at most 8192 rows, 4096 of complex FP64), and 384 KB of
-// entries where they are read every step: R = 16, FP64, 20,800 entries 3.7 us a
-// step (launched 6.1), 31,900 entries 3.3 on short rows (5.0), 39,900 on rows of
-// thirteen 7.3 (6.0); FP32 53,000 entries 5.3 (6.0), 62,400 6.9 (6.2). Rows in
-// registers have no such bound.
-bool onchip_fits(const BsrDev &A, VecMode vm) {
+// Two columns in LDS (at most 8192 rows, about 4,900 of complex FP64). Rows in
+// registers have no other bound. Entries read every step are bound to 384 KB (R =
+// 16, FP64, 20,800 entries 3.7 us a step, launched 6.1; 39,900 on rows of thirteen
+// 7.3, launched 6.0), and cost a step about as much for one column as for 256, where
+// a launched step is 3.6 us for one. Measured, on the chip / launched, us a step: 2,500
+// rows of seven 3.6 / 3.9 (R = 1), 3.8 / 4.8 (16); of thirteen, FP64 5.7 / 4.4, 6.0 / 5.8,
+// FP32 3.5 / 4.3; past 4,096 rows (eight a thread) 4,097 of three 4.1 / 3.6, ragged
+// 4.5 / 4.8 (16), 7,000 of three 5.3 / 3.6, 5.4 / 4.6 (16), 10.9 / 44 (256).
+bool onchip_fits(const BsrDev &A, VecMode vm, int R) {
     if (A.b != 1 || A.is_complex || A.nbr < 1 || A.nbr > 8192 || A.maxlen < 0) return false;
     int rpt, nt;
     onchip_shape((int)A.nbr, &rpt, &nt);
     if (onchip_lds((int)A.nbr, vm, nt) > (size_t)156 << 10) return false;
     const bool held = (A.maxlen <= 4 && rpt <= 4) || (A.maxlen <= 16 && rpt == 1);
-    return held || A.nnzb * (vm.fp32 ? 8 : 12) <= 384 << 10;
+    if (held) return true;
+    if (A.nnzb * (vm.fp32 ? 8 : 12) > 384 << 10) return false;
+    const int row_bytes = R * (vm.complex_vec ? 2 : 1) * (vm.fp32 ? 4 : 8);
+    if (A.nbr > 4096) // FP32 to 6,000 rows of four and five, read together: 4.0 / 4.7 (16)
+        return row_bytes >= 512 || (R >= 16 && ((A.nbr <= 5000 && A.nnzb <= 24000) ||
+                                                (vm.fp32 && A.nbr <= 6000 && A.nnzb >= 4 * A.nbr && A.nnzb <= 5 * A.nbr)));
+    return A.nbr <= 2048 || vm.fp32 || R >= 16 || A.nnzb <= 24000;
 }
 
 hipError_t launch_onchip(const BsrDev &A, VecMode vm, void *t0, void *t1, int R, bool first, int steps,
                          const OnchipWindow &w, double2 *raw, hipStream_t st) {
-    if (!onchip_fits(A, vm) || R < 1 || steps < 0) return hipErrorInvalidValue;
+    if (R < 1 || steps < 0 || !onchip_fits(A, vm, R)) return hipErrorInvalidValue;
     int rpt, nt;
     onchip_shape((int)A.nbr, &rpt, &nt);
     const size_t lds = onchip_lds((int)A.nbr, vm, nt);

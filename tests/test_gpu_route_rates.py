@@ -2,6 +2,8 @@
 kernels, and no slower than the other kernel where its rows are long, short or
 many (kernel times, or wall times of whole runs; each bound lies between the two
 kernels' times)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -94,3 +96,24 @@ def test_long_rows_of_one_lane(monkeypatch):
     with _lib.Context(0):
         pass  # the layout knob is the library's: back to its default
     assert slab <= 1.15 * plain
+
+
+def test_one_column_of_thousands_of_rows(monkeypatch):
+    """7,000 rows of three entries, one column: no slower than replayed launches."""
+    H = neighbours(7000, 1, 1)
+
+    def wall():
+        with _lib.Context(0) as ctx:
+            ctx.upload_bsr(_lib.SLOT_H, H)
+            ctx.set_operator(_lib.FORM_ORTHOGONAL, 0.0, 10.0)
+            ctx.set_samples(7000, 1, _lib.SAMPLES_RADEMACHER, 1)
+            best = 1e9
+            for _ in range(6):
+                t = time.perf_counter()
+                ctx.kpm_moments(2050)
+                best = min(best, time.perf_counter() - t)
+        return best
+
+    default = wall()
+    monkeypatch.setenv("RG_GRAPH", "1")
+    assert default <= 1.2 * wall()
